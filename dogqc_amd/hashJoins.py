@@ -608,6 +608,7 @@ class EquiJoinTranslator(BinaryTranslator):
         while W < pipe.bs * pipe.U:
             W *= 2
         prog = self._prog
+        pipe.sharedAtomics = True
         self.ht["ranked"] = True
         rb = prog.buffer("mmr%d" % J, CType.UINT, pipe.params["n"][1])
         frank = pipe.param("mmr%d" % J, "uint32_t*", "B_" + rb)

@@ -117,7 +117,7 @@ class ExprEmitter(object):
         if pipe.loopOps:
             # rows were reassigned to lanes: no common tile, one search per row
             return "dqc::segment_of(%s, %s, %s[u])" % (f, nb, pipe.tid)
-        return "dqc::segment_of(%s, %s, %s[u], base, %d)" % (f, nb, pipe.tid, pipe.bs * pipe.U)
+        return "dqc::segment_of(%s, %s, %s[u], base + u * step, %d)" % (f, nb, pipe.tid, pipe.bs)
 
     def _MaxExpr(self, e):
         return "std::max<int32_t>(%s, %s)" % (self.emit(e.leftChild), self.emit(e.rightChild))

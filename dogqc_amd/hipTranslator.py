@@ -118,8 +118,15 @@ class Pipeline(object):
     """One generated kernel.
 
     Each thread handles U rows per loop trip (U > 1 only for pipelines
-    without inner loops): row u of trip ``base`` is ``base + u*B + tid``, so
-    for every u a wavefront reads 64 consecutive rows.  Per-row registers are
+    without inner loops), ``step`` rows apart, so for every u a wavefront
+    reads 64 consecutive rows.  A table of at least one full trip of the grid
+    is walked in tiles of U * B consecutive rows per workgroup (step = B); a
+    smaller one in steps of the whole grid, so that its rows reach as many
+    workgroups as there are, instead of U rows on each thread of a few.  Builds
+    wait on their claims, so what counts for them is wavefronts in flight:
+    c1's build of 20 k rows 22.5 -> 14.7 us, c3's item build of 154 k texts
+    38.8 -> 19.1 us.  Steps of the grid at every size cost the streaming
+    kernels (c0 at 64 M rows 446 -> 505 us).  Per-row registers are
     arrays ``name[U]`` indexed by ``u``; all per-row code sits inside
     ``rowLoop()`` blocks, so the U independent rows issue their loads
     together.  When U == 1 the index is the constant ``u = 0``."""
@@ -151,6 +158,7 @@ class Pipeline(object):
         self.dynLdsExpr = None
         self.refillPoints = []
         self.annotations = []
+        self.sharedAtomics = False   # every workgroup updates the same few words
         self.innerDepth = 0
         self.probedJoins = []
         self.nullFlags = {}         # attribute id -> null flag (outer-join build attributes)
@@ -309,24 +317,34 @@ class Pipeline(object):
             else:
                 k.emit("%s %s%s;" % (ct, name, "" if init is None else " = " + init))
         k.extend(self.prologue)
-        if pa is not None:
-            k.emit("const int64_t stride = PHASE == 1 ? (int64_t)%d : (int64_t)gridDim.x * %d;" % (B * U, B * U))
-            k.open("for (int64_t base = PHASE == 1 ? 0 : (int64_t)blockIdx.x * %d;; base += stride)" % (B * U))
+        # lane refills drain their buffers in one more trip, after the last rows
+        end = "" if self.refillPoints else " base < nrows"
+        if U == 1:
+            first, step = "(int64_t)blockIdx.x * %d" % B, "(int64_t)gridDim.x * %d" % B
         else:
-            k.emit("const int64_t stride = (int64_t)gridDim.x * %d;" % (B * U))
-            k.open("for (int64_t base = (int64_t)blockIdx.x * %d;; base += stride)" % (B * U))
+            k.emit("const bool tiled = nrows >= (int64_t)gridDim.x * %d;" % (B * U))
+            first = "(int64_t)blockIdx.x * (tiled ? %d : %d)" % (B * U, B)
+            step = "tiled ? (int64_t)%d : (int64_t)gridDim.x * %d" % (B, B)
+        trip = "(int64_t)gridDim.x * %d" % (B * U)
+        if pa is not None:
+            first, step, trip = ["PHASE == 1 ? %s : %s" % (x, y) for x, y in
+                                 (("0", first), ("(int64_t)%d" % B, step), ("(int64_t)%d" % (B * U), trip))]
+        k.emit("const int64_t step = %s, trip = %s;" % (step, trip))
+        # (lane refills drain their buffers in one more trip, after the last rows)
+        k.open("for (int64_t base = %s;%s; base += trip)" % (first, "" if self.refillPoints else " base < nrows"))
         k.emit("const bool more = base < nrows;")
         k.emit("int active[%d];" % U)
         if U > 1:
             k.emit("#pragma unroll")
             k.open("for (int u = 0; u < %d; ++u)" % U)
-        k.emit("%s[u] = base + (int64_t)(u * %d) + (int64_t)threadIdx.x;" % (self.tid, B))
+        k.emit("%s[u] = base%s + (int64_t)threadIdx.x;" % (self.tid, " + u * step" if U > 1 else ""))
         k.emit("active[u] = more && %s[u] < nrows;" % self.tid)
         if U > 1:
             k.close()
         k.extend(self.code)
         k.extend(self.iterationEnd)
-        k.emit("if (!more) break;")
+        if self.refillPoints:
+            k.emit("if (!more) break;")
         k.close()
         k.extend(self.epilogue)
         k.close()
@@ -561,10 +579,13 @@ class Program(object):
         h.close()
         h.emit("return g_cus;")
         h.close()
-        h.open("static unsigned gridFor(int32_t req, int64_t rows, int bs, int perCu)")
+        h.open("static unsigned gridFor(int32_t req, int64_t rows, int bs, int perCu, int U = 1, int spreadPerCu = 0)")
         h.emit("if (req > 0) return (unsigned)req;")
-        h.emit("int64_t need = (rows + bs - 1) / bs;")
+        h.emit("int64_t need = (rows + (int64_t)bs * U - 1) / ((int64_t)bs * U);")
         h.emit("int64_t cap = (int64_t)computeUnits() * perCu;")
+        h.emit("// below that many workgroups, fewer rows per thread on more of them")
+        h.emit("const int64_t spread = (int64_t)computeUnits() * spreadPerCu;")
+        h.emit("if (need < spread) need = std::min<int64_t>(spread, (rows + bs - 1) / bs);")
         h.emit("int64_t g = std::min<int64_t>(need, cap);")
         h.emit("return (unsigned)std::max<int64_t>(1, g);")
         h.close()
@@ -757,6 +778,12 @@ def pipelineLaunch(prog, pipe, phase=None, rowsExpr=None, perCu=8):
         # an LDS group table is flushed once per workgroup: with many slots,
         # fewer workgroups (8 per CU at <= 512 slots, 1 per CU at >= 4096)
         per = "std::max<int>(1, (int)(%d * 512u / std::max<uint32_t>(512u, L.ldsw[%d])))" % (perCu, pipe.pipeId)
+    # a pipeline whose workgroups each end with (or make per trip) atomics on
+    # shared words spreads a small input over one workgroup per CU, the others
+    # over all that run at once.  One row per thread and up to 2048 workgroups
+    # there took c1's 600 k-slot output kernel (an append) from 14.4 to 30.2 us
+    # and c2's count pass (1 M rows) from 52.8 to 74.5 us.
+    spread = 1 if pipe.sharedAtomics else perCu
     lds = "0" if pipe.dynLdsExpr is None else "(size_t)(%s)" % pipe.dynLdsExpr
     pa = pipe.partAgg
     if pa is not None and phase == 0:
@@ -770,10 +797,10 @@ def pipelineLaunch(prog, pipe, phase=None, rowsExpr=None, perCu=8):
         # the survivors' launch sizes its grid from the queue; the tuned grid
         # belongs to the first launch (with an LDS join filter, a few large
         # workgroups there)
-        lines.append("const unsigned g = gridFor(0, %s, %d, %s);" % (rows, pipe.bs * pipe.U, per))
+        lines.append("const unsigned g = gridFor(0, %s, %d, %s, %d, %d);" % (rows, pipe.bs, per, pipe.U, spread))
     else:
-        lines.append("const unsigned g = gridFor(t->grid[%d] > 0 ? t->grid[%d] : %d, %s, %d, %s);"
-                     % (pipe.pipeId, pipe.pipeId, pipe.defaultGrid, rows, pipe.bs * pipe.U, per))
+        lines.append("const unsigned g = gridFor(t->grid[%d] > 0 ? t->grid[%d] : %d, %s, %d, %s, %d, %d);"
+                     % (pipe.pipeId, pipe.pipeId, pipe.defaultGrid, rows, pipe.bs, per, pipe.U, spread))
     if pa is not None and phase == 0:
         # each workgroup fills its own segment of every partition
         lines[-1] = "const unsigned g = part ? (unsigned)%s : %s;" % (pa["hostNseg"], lines[-1][len("const unsigned g = "):-1])
@@ -1362,6 +1389,7 @@ def materializeRows(ctxt, attrs, isResult, tableName, est, opId):
             pipe.emit("stg%d[wave][sp] = %s;" % (i, c["val"]))
         pipe.code.close()
         pipe.emit("%s += wn;" % wcnt)
+    pipe.sharedAtomics = True
     # final flush, once per workgroup: one global atomic reserves the rows of
     # all its wavefronts' stages (a per-wavefront atomic here serialises
     # thousands of wavefronts on one counter at the end of short kernels)
@@ -1571,6 +1599,7 @@ class AggregationTranslator(UnaryTranslator):
             # LDS, one atomic per workgroup (thousands of atomics on one
             # address serialise at its memory channel)
             nw = pipe.bs // 64
+            pipe.sharedAtomics = True
             for acc in self.accs:
                 red = {"sum": "wave_sum", "count": "wave_sum", "min": "wave_min", "max": "wave_max"}[acc["kind"]]
                 pipe.staticLds.append("__shared__ %s wred%d_%d[%d];" % (acc["ctype"], a.opId, acc["i"], nw))
@@ -1929,6 +1958,7 @@ class AggregationTranslator(UnaryTranslator):
         replicated R times; flushed once per workgroup."""
         pid = pipe.pipeId
         pipe.annotations.append("LDS%d" % self.algExpr.opId)
+        pipe.sharedAtomics = True
         # an estimate beyond 8192 slots turns the tier off, except for keys of
         # a small domain (CHAR, BOOLEAN) without a group-count hint: their
         # groups are often few whatever the input size, so the tier stays

@@ -1,0 +1,59 @@
+"""Row-to-thread mapping of pipelines with several rows per thread: a table of
+at least one full trip of the grid is walked in tiles, a smaller one in steps
+of the whole grid, and both have to reach every row exactly once."""
+import numpy as np
+import pytest
+
+from dogqc_amd import planlib, runtime as rt
+from tests.test_gpu_parity import check, workloadAcc
+
+GRID = 3
+
+
+def walk(n, grid, B, U):
+    """Rows in the order the generated loop assigns them (Pipeline.render)."""
+    tiled = n >= grid * B * U
+    step, trip = (B if tiled else grid * B), grid * B * U
+    out = []
+    for wg in range(grid):
+        base = wg * (B * U if tiled else B)
+        while base < n:
+            for u in range(U):
+                rows = base + u * step + np.arange(B)
+                out.append(rows[rows < n])
+            base += trip
+    return np.concatenate(out) if out else np.zeros(0, int)
+
+
+@pytest.mark.parametrize("U", [1, 2, 4])
+def test_every_row_once(U):
+    B = 8
+    for grid in (1, 3, 4):
+        full = grid * B * U
+        for n in {0, 1, B - 1, B, B + 1, full - 1, full, full + 1, 2 * full - 1, 2 * full, 2 * full + B + 1}:
+            assert np.array_equal(np.sort(walk(n, grid, B, U)), np.arange(n)), (U, grid, n)
+
+
+def test_rendered_mapping():
+    """The generated kernels carry the mapping that `walk` states."""
+    src = planlib.translate("c0").source
+    assert "const bool tiled = nrows >= (int64_t)gridDim.x * 1024;" in src
+    assert "const int64_t step = tiled ? (int64_t)256 : (int64_t)gridDim.x * 256, trip = (int64_t)gridDim.x * 1024;" in src
+    assert "base = (int64_t)blockIdx.x * (tiled ? 1024 : 256); base < nrows; base += trip" in src
+
+
+# one full trip of 3 workgroups x 256 threads x 4 rows is 3072 rows
+@pytest.mark.gpu
+@pytest.mark.parametrize("plan", ["c0", "c1", "c0_batch"])
+@pytest.mark.parametrize("n", [1, 255, 257, 3071, 3072, 3073, 6143, 6145])
+def test_edges(plan, n):
+    t = rt.newTuning()
+    for i in range(rt.MAX_PIPES):
+        t.grid[i] = GRID
+    if plan == "c0_batch":
+        from dogqc_amd import batching
+        acc = workloadAcc("c0", {"cfg0": n}, seed=n)
+        acc = batching.withBatch(acc, {"cfg0": np.array(sorted({max(1, n // 3), max(1, n // 2), n}), dtype=np.int64)})
+    else:
+        acc = workloadAcc(plan, {"cfg0": n} if plan == "c0" else {"dim": n, "fact": n + 5}, seed=n)
+    check(plan, acc, tuning=t, label="n=%d" % n)
