@@ -493,6 +493,51 @@ DQC_DEVICE_INLINE int lds_slot_exact(uint64_t* ltags, uint32_t cap, uint64_t tag
     return -1;
 }
 
+// The front of a workgroup's LDS table: LDS_FRONT slots whose accumulators
+// have many copies, so that the lanes of a wavefront rarely add to one word
+// when a table sized for many groups meets few (or one hot one).  A tag looks
+// at the LDS_FRONT_WINDOW slots from its start slot, read together, and takes
+// the first empty one; -1 when they hold other tags.  Slots are never freed
+// and taken in order, so a tag has one slot or, for good, none.
+constexpr uint32_t LDS_FRONT = 16;
+constexpr uint32_t LDS_FRONT_WINDOW = 4;
+
+DQC_DEVICE_INLINE int lds_front_slot(uint64_t* ftags, uint64_t tag, uint64_t h) {
+    const uint32_t s = slot_of(h, LDS_FRONT - LDS_FRONT_WINDOW + 1u);
+    for (;;) {
+        uint64_t t[LDS_FRONT_WINDOW];
+#pragma unroll
+        for (uint32_t i = 0; i < LDS_FRONT_WINDOW; ++i)
+            t[i] = __hip_atomic_load(&ftags[s + i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        int hit = -1, empty = -1;
+#pragma unroll
+        for (int i = (int)LDS_FRONT_WINDOW - 1; i >= 0; --i) {
+            if (t[i] == tag) hit = i;
+            if (t[i] == TAG_EMPTY) empty = i;
+        }
+        if (hit >= 0) return (int)s + hit;
+        if (empty < 0) return -1;
+        uint64_t expected = TAG_EMPTY;
+        if (__hip_atomic_compare_exchange_strong(&ftags[s + empty], &expected, tag, __ATOMIC_RELAXED,
+                                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) ||
+            expected == tag)
+            return (int)s + empty;
+    }
+}
+
+// Accumulator copy of a row's group in a workgroup's LDS table: the front
+// (nf slots, 0 without one, rf copies each), then w slots of r copies each;
+// -1 when the group has no slot.  Copy counts are powers of two.
+DQC_DEVICE_INLINE int lds_entry(uint64_t* ltags, uint32_t nf, uint32_t rf, uint32_t w, uint32_t r, uint64_t tag,
+                                uint64_t h) {
+    if (nf) {
+        const int f = lds_front_slot(ltags, tag, h);
+        if (f >= 0) return f * (int)rf + (int)(lane_id() & (rf - 1u));
+    }
+    const int s = lds_slot_exact(ltags + nf, w, tag, h);
+    return s < 0 ? -1 : (int)(nf * rf) + s * (int)r + (int)(lane_id() & (r - 1u));
+}
+
 // ------------------------------------------------------ join filter
 // Blocked Bloom filter of a unique join's build keys: `words` 32-bit words
 // (a power of two), two bits of one word per key, all from the key's hash.

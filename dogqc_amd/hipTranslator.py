@@ -37,7 +37,6 @@ from dogqc_amd.kernel import KernelCall
 from dogqc_amd.util import listWrap
 
 WAVE = 64
-LDS_AGG_BUDGET = 48 * 1024
 
 
 def _pow2ceil(x):
@@ -131,11 +130,11 @@ class Pipeline(object):
     ``rowLoop()`` blocks, so the U independent rows issue their loads
     together.  When U == 1 the index is the constant ``u = 0``."""
 
-    def __init__(self, program, name, source, U=1):
+    def __init__(self, program, name, source, U=1, bs=None):
         self.program = program
         self.name = name
         self.pipeId = len(program.pipes)
-        self.bs = int(KernelCall.defaultBlockSize)
+        self.bs = int(bs or KernelCall.defaultBlockSize)
         if self.bs % WAVE or not (WAVE <= self.bs <= 1024):
             raise ValueError("block size must be a multiple of 64 in [64, 1024]")
         self.U = max(1, int(U))
@@ -158,6 +157,7 @@ class Pipeline(object):
         self.dynLdsExpr = None
         self.refillPoints = []
         self.annotations = []
+        self.fewGroups = False       # ends in a group-by known to have few groups (launchShape)
         self.sharedAtomics = False   # every workgroup updates the same few words
         self.innerDepth = 0
         self.probedJoins = []
@@ -433,10 +433,11 @@ class Program(object):
         self.hts.append(rec)
         return rec
 
-    def newPipeline(self, name, source, U=1):
+    def newPipeline(self, name, source, U=1, bs=None, wide=False):
         if len(self.pipes) >= 32:
             raise ValueError("too many pipelines in one plan")
-        pipe = Pipeline(self, name, source, U)
+        pipe = Pipeline(self, name, source, U, bs)
+        pipe.wide = wide
         self.pipes.append(pipe)
         return pipe
 
@@ -544,6 +545,7 @@ class Program(object):
         h.emit("    int64_t rows[%d];" % max(1, nt))
         h.emit("    uint32_t ldsw[%d];" % max(1, len(self.pipes)))
         h.emit("    uint32_t ldsr[%d];" % max(1, len(self.pipes)))
+        h.emit("    uint32_t ldsf[%d];" % max(1, len(self.pipes)))
         h.emit("    uint32_t arep[%d];" % max(1, len(self.hts)))
         h.emit("    uint32_t apart[%d];" % max(1, len(self.hts)))
         h.emit("    uint32_t apbits[%d];" % max(1, len(self.hts)))
@@ -776,8 +778,11 @@ def pipelineLaunch(prog, pipe, phase=None, rowsExpr=None, perCu=8):
     per = str(perCu)
     if "lw" in pipe.params:
         # an LDS group table is flushed once per workgroup: with many slots,
-        # fewer workgroups (8 per CU at <= 512 slots, 1 per CU at >= 4096)
+        # fewer workgroups (8 per CU at <= 512 slots, 1 per CU at >= 4096), and
+        # one of the few-groups shape per CU (launchShape)
         per = "std::max<int>(1, (int)(%d * 512u / std::max<uint32_t>(512u, L.ldsw[%d])))" % (perCu, pipe.pipeId)
+        if pipe.fewGroups:
+            per = "1"
     # a pipeline whose workgroups each end with (or make per trip) atomics on
     # shared words spreads a small input over one workgroup per CU, the others
     # over all that run at once.  One row per thread and up to 2048 workgroups
@@ -790,7 +795,7 @@ def pipelineLaunch(prog, pipe, phase=None, rowsExpr=None, perCu=8):
         # rows are scattered to partitions: no LDS group table in this pass
         lines.append("const bool part = %s > 0u;" % pa["hostNp"])
         if "lw" in pipe.params:
-            lines.append("if (part) kp.lw = 0u;")
+            lines.append("if (part) { kp.lw = 0u; kp.lf = 0u; }")
         keep = "(size_t)0" if pipe.ldsFilter is None else "(size_t)(%s)" % pipe.ldsFilter["host"]
         lds = "(part ? %s : %s)" % (keep, lds)
     if phase == 1 and getattr(pipe, "globalRefill", False):
@@ -801,6 +806,13 @@ def pipelineLaunch(prog, pipe, phase=None, rowsExpr=None, perCu=8):
     else:
         lines.append("const unsigned g = gridFor(t->grid[%d] > 0 ? t->grid[%d] : %d, %s, %d, %s, %d, %d);"
                      % (pipe.pipeId, pipe.pipeId, pipe.defaultGrid, rows, pipe.bs, per, pipe.U, spread))
+    if pipe.fewGroups:
+        # rows enough for a workgroup to be worth its flush, every group of
+        # its table: 8 per slot (a 246 k-row, 175-group group-by
+        # 41 us at 240 workgroups, 25 us at 61)
+        lines[-1] = lines[-1].replace("const unsigned g", "unsigned g")
+        lines.append("if (t->grid[%d] <= 0) g = (unsigned)std::max<int64_t>(1, std::min<int64_t>(g, (%s) / "
+                     "(8 * (int64_t)std::min<uint32_t>(512u, L.ldsw[%d]) + 1)));" % (pipe.pipeId, rows, pipe.pipeId))
     if pa is not None and phase == 0:
         # each workgroup fills its own segment of every partition
         lines[-1] = "const unsigned g = part ? (unsigned)%s : %s;" % (pa["hostNseg"], lines[-1][len("const unsigned g = "):-1])
@@ -1061,6 +1073,47 @@ def rowsPerThread(translator):
     return 1 if loops else max(1, int(KernelCall.defaultRowsPerThread))
 
 
+def launchShape(translator):
+    """(rows per thread, block size, few groups) of the pipeline a scan opens.
+
+    A pipeline that ends in a group-by known to have few groups takes four
+    times the block (at most 1024 threads, the rows per thread cut to match),
+    one workgroup per CU: every workgroup flushes all its groups with
+    device-scope atomics on the same few words, about 10 G/s over the chip,
+    so the fewer and larger the workgroups the better.  At 256 x 4 and 8 per
+    CU against 1024 x 1 and 1 per CU: c0 at 1 M rows 49.8 -> 14.6 us, at 64 M
+    446 -> 357 us (6.1 TB/s); 3.2 M rows into 175 groups 157 -> 44 us.  (Two
+    rows per thread: 64 M-row c0 379 us, TPC-H Q1 at SF10 268 instead of
+    273 us.)"""
+    U, B = rowsPerThread(translator), int(KernelCall.defaultBlockSize)
+    if pipelineShape(translator)[0] or not _fewGroupsAbove(translator):
+        return U, B, False
+    wide = min(1024, 4 * B)
+    return max(1, U * B // wide), wide, True
+
+
+def _fewGroupsAbove(translator):
+    """The pipeline ends in a group-by known to have few groups (a hint, or
+    keys of a small domain) whose keys pack into an exact tag."""
+    t = translator
+    while t.parent is not None:
+        p = t.parent
+        if isinstance(p, BinaryTranslator) and p.leftChild is t:
+            return False
+        if isinstance(p, AggregationTranslator):
+            a = p.algExpr
+            groups = list(a.groupAttributes.values()) if a.doGroup else []
+            if not groups or sum(_GROUP_BITS.get(g.dataType, 65) for g in groups) > 64:
+                return False
+            if getattr(a, "numgroupsFromCfg", False):
+                return a.numgroups <= 4096
+            return _keyDomain(groups) is not None
+        if isinstance(p, MaterializeTranslator):
+            return False
+        t = p
+    return False
+
+
 class ScanTranslator(LiteralTranslator):
     """Opens a pipeline over a base table.  Columns load lazily at first use,
     except those whose cache lines would nearly all be read anyway: a column
@@ -1085,7 +1138,7 @@ class ScanTranslator(LiteralTranslator):
             return
         ti = prog.table(tname)
         pipe = prog.newPipeline(name, {"rows": "L.rows[%d]" % ti, "tidName": "%s%d" % (tname, a.scanTableId)},
-                                rowsPerThread(self))
+                                *launchShape(self))
         pipe.scanTable = tname
         ctxt.pipe = pipe
         tid = pipe.tid + "[u]"
@@ -1136,7 +1189,7 @@ class ScanTranslator(LiteralTranslator):
             raise ValueError("temp table %s is scanned before it is created" % a.table["name"])
         ti = tmp["index"]
         pipe = prog.newPipeline(name, {"rows": "L.tcap[%d]" % ti, "devRows": "st->temp_count[%d]" % ti,
-                                       "tidName": "%s%d" % (a.table["name"], a.scanTableId)}, rowsPerThread(self))
+                                       "tidName": "%s%d" % (a.table["name"], a.scanTableId)}, *launchShape(self))
         ctxt.pipe = pipe
         tid = pipe.tid + "[u]"
         byName = {c["name"]: c for c in tmp["columns"]}
@@ -1495,9 +1548,14 @@ class AggregationTranslator(UnaryTranslator):
       * grouping with keys that pack into an exact tag (63 bits with the
         top bit set, or exactly 64 bits stored as key + 1 with the single
         key whose tag would be 0 kept in an extra slot at index cap): a workgroup
-        LDS table of W tag slots whose accumulators are replicated R times
-        (lane i uses replica i mod R, so lanes of one wavefront rarely hit the
-        same LDS word), flushed to the global table once per workgroup; rows
+        LDS table of W tag slots, flushed to the global table once per
+        workgroup.  Lanes of one wavefront that add to the same LDS word take
+        turns, so accumulators have copies (lane i uses copy i mod R): 16 in
+        a table of 16 slots, and in the 16-slot front (dqc::lds_front_slot)
+        that a table of up to 512 slots has before its slots of one copy,
+        whose groups are many enough to spread the lanes.  TPC-H Q1 is hinted
+        100 groups and has 4: 256 slots of 4 copies ran 400 us at SF10, with
+        the front 273 us; rows
         whose group does not fit the LDS table go straight to the global
         table;
       * other keys: the global table in hashed mode.
@@ -1718,14 +1776,11 @@ class AggregationTranslator(UnaryTranslator):
             pipe.code.open("if (active[u])")
             pipe.emit("%s = %s;" % (gtag, tagCode))
             pipe.emit("const uint64_t gh = dqc::mix64(%s);" % gtag)
-            pipe.emit("int ls = -1;")
-            if self.exact64:
-                # tag 0 (key ~0) bypasses the LDS table and uses slot cap
-                pipe.emit("if (p.lw && %s != 0) ls = dqc::lds_slot_exact(ltags, p.lw, %s, %s);" % (gtag, gtag, ldsHash))
-            else:
-                pipe.emit("if (p.lw) ls = dqc::lds_slot_exact(ltags, p.lw, %s, %s);" % (gtag, ldsHash))
-            pipe.code.open("if (ls >= 0)")
-            pipe.emit("const uint32_t li = (uint32_t)ls * p.lr + (lane & (p.lr - 1u));")
+            pipe.emit("int li = -1;")
+            # (64-bit keys: tag 0, key ~0, bypasses the LDS table and uses slot cap)
+            pipe.emit("if (p.lw%s) li = dqc::lds_entry(ltags, p.lf, p.lfr, p.lw, p.lr, %s, %s);"
+                      % (" && %s != 0" % gtag if self.exact64 else "", gtag, ldsHash))
+            pipe.code.open("if (li >= 0)")
             for acc, v in zip(self.accs, vals):
                 pipe.emit(_guarded(acc, _ldsOp(acc["kind"], "&lacc%d[li]" % acc["i"], v)))
             pipe.code.close()
@@ -1761,6 +1816,10 @@ class AggregationTranslator(UnaryTranslator):
             pipe.code.close()
             pipe.emit(upd["overflow"])
             pipe.code.close()
+
+    # copies of a group's accumulators in the LDS table's front (and in a table
+    # of at most LDS_FRONT slots)
+    LDS_COPIES = 16
 
     # partitioned group-by: at most this many partitions and first-pass
     # workgroups (segments per partition); auto mode above this many groups
@@ -1959,6 +2018,7 @@ class AggregationTranslator(UnaryTranslator):
         pid = pipe.pipeId
         pipe.annotations.append("LDS%d" % self.algExpr.opId)
         pipe.sharedAtomics = True
+        pipe.fewGroups = pipe.wide and pipe.partAgg is None
         # an estimate beyond 8192 slots turns the tier off, except for keys of
         # a small domain (CHAR, BOOLEAN) without a group-count hint: their
         # groups are often few whatever the input size, so the tier stays
@@ -1973,55 +2033,73 @@ class AggregationTranslator(UnaryTranslator):
         if pipe.ldsFilter is not None:
             used = "(%s + %s)" % (used, pipe.ldsFilter["host"])
             devBase, hostBase = pipe.ldsFilter["dev"], pipe.ldsFilter["host"]
+        fits = "(uint64_t)F * (8u + (uint64_t)FR * %du) + (uint64_t)W * (8u + (uint64_t)R * %du) + %s <= maxLds()" % (
+            accBytes, accBytes, used)
         prog.hostVars["lds%d" % pid] = (
-            "{ int64_t w = t->lds_slots[%d]; uint32_t W = 0, R = 1;\n"
+            "{ int64_t w = t->lds_slots[%d]; uint32_t W = 0, R = 1, F = 0, FR = 1;\n"
             "  if (w > 0) W = pow2floor((uint64_t)w);\n"
             "  else if (w == 0) W = std::max<uint32_t>(16u, pow2ceil((uint64_t)std::max<int64_t>(1, %s) * 2u));\n"
             "  if (W > 8192u) W = %s;\n"
             "  W = std::min<uint32_t>(W, 4096u);\n"
             "  if (W) {\n"
-            "    int64_t r = t->lds_replicas[%d];\n"
+            "    const int64_t r = t->lds_replicas[%d];\n"
             "    if (r > 0) R = std::min<uint32_t>(64u, pow2floor((uint64_t)r));\n"
-            "    else { R = 64u; while (R > 1u && (uint64_t)W * (8u + (uint64_t)R * %du) > %du) R /= 2u; }\n"
-            "    while (W > 16u && (uint64_t)W * (8u + (uint64_t)R * %du) + %s > maxLds()) W /= 2u;\n"
-            "    if ((uint64_t)W * (8u + (uint64_t)R * %du) + %s > maxLds()) W = 0;\n"
+            "    else if (W <= dqc::LDS_FRONT) R = %du;\n"
+            "    else if (W <= 512u || %s) { F = dqc::LDS_FRONT; FR = %du; }\n"
+            "    while (W > 16u && !(%s)) W /= 2u;\n"
+            "    if (!(%s)) F = 0u;\n"
+            "    if (!(%s)) W = 0;\n"
             "  }\n"
-            "  L.ldsw[%d] = W; L.ldsr[%d] = W ? R : 1u; }"
-            % (pid, est, overflowW, pid, accBytes, LDS_AGG_BUDGET, accBytes, used, accBytes, used, pid, pid))
+            "  L.ldsw[%d] = W; L.ldsr[%d] = W ? R : 1u; L.ldsf[%d] = W ? F : 0u; }"
+            % (pid, est, overflowW, pid, self.LDS_COPIES, "true" if bounded else "false", self.LDS_COPIES,
+               fits, fits, fits, pid, pid, pid))
         pipe.param("lw", "uint32_t", "L.ldsw[%d]" % pid)
         pipe.param("lr", "uint32_t", "L.ldsr[%d]" % pid)
+        pipe.param("lf", "uint32_t", "L.ldsf[%d]" % pid)
+        pipe.param("lfr", "uint32_t", "%du" % self.LDS_COPIES)
         # dynamic LDS: tags, then one region per accumulator (8-byte aligned)
-        parts = ["(uint64_t)L.ldsw[%d] * 8u" % pid]
+        entries = "((uint64_t)L.ldsf[%d] * %du + (uint64_t)L.ldsw[%d] * L.ldsr[%d])" % (pid, self.LDS_COPIES, pid, pid)
+        parts = ["(uint64_t)(L.ldsf[%d] + L.ldsw[%d]) * 8u" % (pid, pid)]
         for acc in self.accs:
-            parts.append("(((uint64_t)L.ldsw[%d] * L.ldsr[%d] * %d + 7u) & ~(uint64_t)7u)"
-                         % (pid, pid, CType.size[acc["ctype"]]))
+            parts.append("((%s * %d + 7u) & ~(uint64_t)7u)" % (entries, CType.size[acc["ctype"]]))
         if hostBase is not None:
             parts.insert(0, hostBase)
         pipe.dynLdsExpr = " + ".join(parts)
         pro = pipe.prologue
         pro.emit("uint64_t* ltags = (uint64_t*)(dqc_dyn_lds + %s);" % devBase)
-        pro.emit("uint64_t loff = %s + (uint64_t)p.lw * 8u;" % devBase)
+        pro.emit("const uint32_t lent = p.lf * p.lfr + p.lw * p.lr;")
+        pro.emit("uint64_t loff = %s + (uint64_t)(p.lf + p.lw) * 8u;" % devBase)
         for acc in self.accs:
             pro.emit("%s* lacc%d = (%s*)(dqc_dyn_lds + loff);" % (acc["ctype"], acc["i"], acc["ctype"]))
-            pro.emit("loff += ((uint64_t)p.lw * p.lr * %d + 7u) & ~(uint64_t)7u;" % CType.size[acc["ctype"]])
-        pro.emit("for (uint32_t i = threadIdx.x; i < p.lw; i += %du) ltags[i] = 0;" % pipe.bs)
-        pro.open("for (uint32_t i = threadIdx.x; i < p.lw * p.lr; i += %du)" % pipe.bs)
+            pro.emit("loff += ((uint64_t)lent * %d + 7u) & ~(uint64_t)7u;" % CType.size[acc["ctype"]])
+        pro.emit("for (uint32_t i = threadIdx.x; i < p.lf + p.lw; i += %du) ltags[i] = 0;" % pipe.bs)
+        pro.open("for (uint32_t i = threadIdx.x; i < lent; i += %du)" % pipe.bs)
         for acc in self.accs:
             pro.emit("lacc%d[i] = %s;" % (acc["i"], _cIdentity(acc["kind"], acc["ctype"])))
         pro.close()
         pro.emit("__syncthreads();")
+        # one lane per copy (a slot's copies are consecutive lanes, and the
+        # front is a multiple of 64 copies, so a wavefront sees one copy
+        # count): an exchange folds them, the slot's first lane updates the
+        # global table
         ep = pipe.epilogue
         ep.emit("__syncthreads();")
-        # few replicas: one thread per slot folds them; many: one wavefront
-        # per slot reduces them across lanes
-        ep.open("if (p.lr < 16u)")
-        ep.open("for (uint32_t s = threadIdx.x; s < p.lw; s += %du)" % pipe.bs)
-        ep.emit("const uint64_t tg = ltags[s];")
-        ep.emit("if (tg == 0) continue;")
+        ep.open("for (uint32_t e0 = wave * 64u; e0 < lent; e0 += %du)" % pipe.bs)
+        ep.emit("const uint32_t e = e0 + lane;")
+        ep.emit("const bool front = e0 < p.lf * p.lfr;")
+        ep.emit("const uint32_t r = front ? p.lfr : p.lr;")
+        ep.emit("const uint32_t s = front ? e / p.lfr : p.lf + (e - p.lf * p.lfr) / p.lr;")
+        ep.emit("const uint64_t tg = e < lent ? ltags[s] : 0ull;")
+        ep.emit("if (dqc::ballot(tg != 0ull) == 0ull) continue;")
         for acc in self.accs:
-            ep.emit("%s f%d = lacc%d[s * p.lr];" % (acc["ctype"], acc["i"], acc["i"]))
-            ep.emit("for (uint32_t r = 1; r < p.lr; ++r) { const %s v = lacc%d[s * p.lr + r]; %s }"
+            ep.emit("%s f%d = e < lent ? lacc%d[e] : %s;" % (acc["ctype"], acc["i"], acc["i"],
+                                                            _cIdentity(acc["kind"], acc["ctype"])))
+        ep.open("for (uint32_t d = 1; d < r; d <<= 1)")
+        for acc in self.accs:
+            ep.emit("{ const %s v = __shfl_xor(f%d, (int)d, 64); %s }"
                     % (acc["ctype"], acc["i"], _combine(acc["kind"], "f%d" % acc["i"], "v")))
+        ep.close()
+        ep.open("if (tg != 0ull && (e & (r - 1u)) == 0u)")
         ep.emit("const int64_t gs = dqc::agg_slot_exact(%s, %s, tg, dqc::mix64(tg), &st->flags);" % (ftags, fcap))
         ep.open("if (gs >= 0)")
         for acc in self.accs:
@@ -2029,26 +2107,6 @@ class AggregationTranslator(UnaryTranslator):
         ep.close()
         ep.emit("else { dqc::raise_status(&st->flags, DQC_ST_HT_OVERFLOW); atomicOr(&st->ht_overflow_mask, %du); }"
                 % (1 << self.ht["index"]))
-        ep.close()
-        ep.close()
-        ep.open("else")
-        ep.open("for (uint32_t s = wave; s < p.lw; s += %du)" % (pipe.bs // WAVE))
-        ep.emit("const uint64_t tg = ltags[s];")
-        ep.emit("if (tg == 0) continue;")
-        for acc in self.accs:
-            red = {"sum": "wave_sum", "count": "wave_sum", "min": "wave_min", "max": "wave_max"}[acc["kind"]]
-            ep.emit("%s f%d = lane < p.lr ? lacc%d[s * p.lr + lane] : %s;" % (
-                acc["ctype"], acc["i"], acc["i"], _cIdentity(acc["kind"], acc["ctype"])))
-            ep.emit("f%d = dqc::%s(f%d);" % (acc["i"], red, acc["i"]))
-        ep.open("if (lane == 0)")
-        ep.emit("const int64_t gs = dqc::agg_slot_exact(%s, %s, tg, dqc::mix64(tg), &st->flags);" % (ftags, fcap))
-        ep.open("if (gs >= 0)")
-        for acc in self.accs:
-            ep.emit("%s;" % _atomic(acc["kind"], "%s[%s + gs]" % (acc["field"], aoff), "f%d" % acc["i"]))
-        ep.close()
-        ep.emit("else { dqc::raise_status(&st->flags, DQC_ST_HT_OVERFLOW); atomicOr(&st->ht_overflow_mask, %du); }"
-                % (1 << self.ht["index"]))
-        ep.close()
         ep.close()
         ep.close()
 
@@ -2061,7 +2119,7 @@ class AggregationTranslator(UnaryTranslator):
         rows = "L.htcap[%d]" % (self.fused["htIndex"] if self.fused else self.ht["index"])
         if (self.fused is None and self.doGroup and self.exact64) or (self.fused is not None and self.fused["tag32"]):
             rows += " + 1"     # the extra slot
-        pipe = prog.newPipeline(name, {"rows": rows, "tidName": "agg%d" % a.opId}, rowsPerThread(self))
+        pipe = prog.newPipeline(name, {"rows": rows, "tidName": "agg%d" % a.opId}, *launchShape(self))
         ctxt.pipe = pipe
         tid = pipe.tid + "[u]"
         pipe.param("st", "dqc_plan_status*", "st")

@@ -57,3 +57,15 @@ def test_edges(plan, n):
     else:
         acc = workloadAcc(plan, {"cfg0": n} if plan == "c0" else {"dim": n, "fact": n + 5}, seed=n)
     check(plan, acc, tuning=t, label="n=%d" % n)
+
+
+# the LDS table's 16-slot front: fewer groups than it has slots, as many, more,
+# and the key (-1, -1) whose 64-bit tag is 0 and bypasses the LDS table
+@pytest.mark.gpu
+@pytest.mark.parametrize("groups", [1, 2, 13, 16, 17, 60, 128])
+@pytest.mark.parametrize("n", [1, 1025, 70001])
+def test_front_table(groups, n):
+    acc = planlib.featureData(n, 10, seed=groups)
+    acc.data[("t", "t_grp")] = (np.arange(n) % groups - 1).astype(np.int32)
+    check("f_groupby_64", acc, label="groups=%d n=%d" % (groups, n))
+    check("f_groupby_wide", acc, label="groups=%d n=%d" % (groups, n))
