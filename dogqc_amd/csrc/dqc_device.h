@@ -147,6 +147,20 @@ DQC_DEVICE_INLINE uint32_t slot_of(uint64_t h, uint32_t cap) {
     return (uint32_t)(((h >> 32) * (uint64_t)cap) >> 32);
 }
 
+// Hash of a key of at most 32 bits: the 32-bit finaliser of MurmurHash3
+// (Austin Appleby, public domain) in the upper half, which picks the slot, and
+// one more multiple of it in the lower half for the join filter.  Probes of
+// streamed rows are bound by their VALU instructions, and this costs 3
+// quarter-rate multiplies where mix64 costs 8.
+DQC_DEVICE_INLINE uint64_t hash32(uint32_t k) {
+    k ^= k >> 16;
+    k *= 0x85ebca6bu;
+    k ^= k >> 13;
+    k *= 0xc2b2ae35u;
+    k ^= k >> 16;
+    return ((uint64_t)k << 32) | (uint64_t)(k * 0x9e3779b1u);
+}
+
 DQC_DEVICE_INLINE uint32_t next_slot(uint32_t s, uint32_t cap) { return (s + 1u == cap) ? 0u : s + 1u; }
 
 // ------------------------------------------------------------ status word
@@ -185,13 +199,40 @@ DQC_DEVICE_INLINE Tag cas_tag(Tag* p, Tag expected, Tag desired) {
     return expected;
 }
 
+// Slots a claim that found its home slot taken looks at together: one memory
+// round trip instead of one per slot, until a wavefront's last lane is done
+// (200 k keys 30.9 -> 24.1 us; the group tables' claims, whose first slot is
+// nearly always the right one, got slower with it and go slot by slot).
+constexpr uint32_t WALK = 4;
+
+// The WALK tags from slot s on as other workgroups have left them (agent
+// scope); slots at or past cap are slot s again.
+template <typename Tag>
+DQC_DEVICE_INLINE void walk_load(const Tag* tags, uint32_t s, uint32_t cap, Tag (&t)[WALK]) {
+#pragma unroll
+    for (uint32_t i = 0; i < WALK; ++i)
+        t[i] = __hip_atomic_load(&tags[s + i < cap ? s + i : s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 template <typename Tag>
 DQC_DEVICE_INLINE int64_t ht_insert_from(Tag* tags, uint32_t cap, Tag tag, uint32_t s, uint32_t n,
                                          const uint32_t* status) {
-    for (; n < cap && n < MAX_PROBE; ++n) {
-        if ((n & 31u) == 31u && overflow_raised(status)) return -1;
-        if (cas_tag(&tags[s], (Tag)TAG_EMPTY, tag) == (Tag)TAG_EMPTY) return (int64_t)s;
-        s = next_slot(s, cap);
+    while (n < cap && n < MAX_PROBE) {
+        if (n >= 32u && overflow_raised(status)) return -1;
+        Tag t[WALK];
+        walk_load(tags, s, cap, t);
+        const uint32_t left = cap - s < WALK ? cap - s : WALK;
+        uint32_t k = left;      // the first empty slot of the window
+#pragma unroll
+        for (uint32_t i = WALK; i-- > 0u;)
+            if (i < left && t[i] == (Tag)TAG_EMPTY) k = i;
+        if (k < left) {
+            if (n + k >= cap || n + k >= MAX_PROBE) return -1;
+            if (cas_tag(&tags[s + k], (Tag)TAG_EMPTY, tag) == (Tag)TAG_EMPTY) return (int64_t)(s + k);
+            ++k;                // taken since: go on after it
+        }
+        n += k;
+        s = s + k >= cap ? 0u : s + k;
     }
     return -1;
 }
@@ -201,23 +242,8 @@ DQC_DEVICE_INLINE int64_t ht_insert(uint64_t* tags, uint32_t cap, uint64_t tag, 
     return ht_insert_from<uint64_t>(tags, cap, tag, slot_of(h, cap), 0u, status);
 }
 
-// Find the next slot holding `tag`, starting at *cursor (initialise the
-// cursor with probe_start).  Returns -1 at the first empty slot or after a
-// full cycle.  Used by join probes, which run after the build kernel ended.
+// A join probe starts here.
 DQC_DEVICE_INLINE uint32_t probe_start(uint64_t h, uint32_t cap) { return slot_of(h, cap); }
-
-template <typename Tag>
-DQC_DEVICE_INLINE int64_t ht_probe(const Tag* tags, uint32_t cap, Tag tag, uint32_t& cursor, uint32_t& visited) {
-    while (visited < cap && visited < MAX_PROBE) {
-        uint32_t s = cursor;
-        const Tag t = tags[s];
-        cursor = next_slot(s, cap);
-        ++visited;
-        if (t == tag) return (int64_t)s;
-        if (t == (Tag)TAG_EMPTY) { visited = cap; return -1; }
-    }
-    return -1;
-}
 
 // A group's accumulator combined over its R copies (copy r at a[i + r*stride];
 // global group-by tables keep one copy per XCD-sized group of workgroups).
@@ -249,15 +275,15 @@ DQC_DEVICE_INLINE T rep_max(const T* a, int64_t i, uint32_t R, uint64_t stride) 
 }
 
 // The next PROBE_WINDOW slots s, s+1, ... of a unique join table, read with
-// 16-byte loads (two for 64-bit tags, one for 32-bit tags) so one memory
+// 16-byte loads (two for 64-bit slots, one for 32-bit tags) so one memory
 // round trip resolves most probes, hits and misses alike.  Join tag buffers
 // carry PROBE_WINDOW padding slots (the 32-bit extra slot included) so the
-// window never leaves the allocation; slots at or past cap are ignored.
+// window never leaves the allocation; slots at or past cap are not looked at.
 constexpr uint32_t PROBE_WINDOW = 4;
 
-template <typename Tag>
+template <typename Slot>
 struct probe_win {
-    Tag t[PROBE_WINDOW];
+    Slot t[PROBE_WINDOW];
 };
 
 DQC_DEVICE_INLINE probe_win<uint64_t> probe_window(const uint64_t* tags, uint32_t s) {
@@ -283,29 +309,6 @@ DQC_DEVICE_INLINE probe_win<uint32_t> probe_window(const uint32_t* tags, uint32_
     return w;
 }
 
-// Resolve a probe from its window: the slot holding `tag` (>= 0), -1 when an
-// empty slot comes first, -2 when every window slot holds another tag; then
-// the probe continues with ht_probe at `cursor` with `visited` slots tried.
-template <typename Tag>
-DQC_DEVICE_INLINE int64_t probe_in_window(const probe_win<Tag>& w, uint32_t s, uint32_t cap, Tag tag,
-                                          uint32_t& cursor, uint32_t& visited) {
-    int64_t r = -2;
-    uint32_t n = 0;
-#pragma unroll
-    for (uint32_t i = 0; i < PROBE_WINDOW; ++i) {
-        if (r == -2 && s + i < cap) {
-            ++n;
-            if (w.t[i] == tag)
-                r = (int64_t)(s + i);
-            else if (w.t[i] == (Tag)TAG_EMPTY)
-                r = -1;
-        }
-    }
-    visited = n;
-    cursor = s + n >= cap ? 0u : s + n;
-    return r;
-}
-
 // Packed unique tables: a key packing into 32 bits with one stored column of
 // at most 4 bytes keeps both in one 64-bit slot, the tag (packed key + 1) in
 // the low half and the column's bits in the high half, so a probe that finds
@@ -324,36 +327,75 @@ DQC_DEVICE_INLINE T packed_payload(uint64_t slot) {
     return v;
 }
 
-// probe_in_window over packed slots: the low halves hold the tags
-DQC_DEVICE_INLINE int64_t probe_in_window_packed(const probe_win<uint64_t>& w, uint32_t s, uint32_t cap,
-                                                 uint32_t tag, uint32_t& cursor, uint32_t& visited) {
-    int64_t r = -2;
-    uint32_t n = 0;
+// What a window of slots says about `tag` (not 0), looked up in one of the
+// slots from its home slot on: the index of the first slot that holds it, or
+// PROBE_WINDOW; `empty` when some slot is empty.  Slots are claimed in order
+// from the home slot and never freed, so a tag that is in the table has no
+// empty slot before it: with an empty slot in the window and no hit, it is
+// absent.  A slot word's tag is its low half where words are packed slots.
+//
+// VALU instructions bound the probes of streamed rows: c3's sales kernel spent
+// 493 a wavefront and trip (60 M rows, 462 M in all, 1155 us), most of them in
+// 64-bit slot bookkeeping per window slot, in mix64 and in a walk of one slot
+// and memory round trip at a time for the lanes (1 in 8 at a load of one half)
+// whose window does not decide.  With hash32, this window test and a walk by
+// windows it takes 762 us, TPC-H Q3's two probing kernels 125 -> 85 us.
+template <typename Slot, typename Tag>
+DQC_DEVICE_INLINE uint32_t window_find(const probe_win<Slot>& w, Tag tag, bool& empty) {
+    uint32_t k = PROBE_WINDOW;
+    Tag least = (Tag)w.t[0];
 #pragma unroll
-    for (uint32_t i = 0; i < PROBE_WINDOW; ++i) {
-        if (r == -2 && s + i < cap) {
-            ++n;
-            if ((uint32_t)w.t[i] == tag)
-                r = (int64_t)(s + i);
-            else if (w.t[i] == 0ull)
-                r = -1;
-        }
+    for (uint32_t i = PROBE_WINDOW; i-- > 0u;) {
+        k = (Tag)w.t[i] == tag ? i : k;
+        least = (Tag)w.t[i] < least ? (Tag)w.t[i] : least;
     }
-    visited = n;
-    cursor = s + n >= cap ? 0u : s + n;
-    return r;
+    empty = least == (Tag)0;
+    return k;
 }
 
-// ht_probe over packed slots
-DQC_DEVICE_INLINE int64_t ht_probe_packed(const uint64_t* slots, uint32_t cap, uint32_t tag, uint32_t& cursor,
-                                          uint32_t& visited) {
+// Resolve a probe from the window at its home slot s: the slot holding `tag`,
+// -1 when it is absent, -2 when every window slot holds another tag or the
+// window reaches past the table's end; then the probe goes on with ht_probe
+// at `cursor` with `visited` slots tried.
+template <typename Slot, typename Tag>
+DQC_DEVICE_INLINE int64_t probe_in_window(const probe_win<Slot>& w, uint32_t s, uint32_t cap, Tag tag,
+                                          uint32_t& cursor, uint32_t& visited) {
+    bool empty;
+    const uint32_t k = window_find(w, tag, empty);
+    const bool whole = cap >= PROBE_WINDOW && s <= cap - PROBE_WINDOW;
+    visited = whole ? PROBE_WINDOW : 0u;
+    cursor = s + visited;       // == cap: ht_probe wraps
+    const int64_t missed = empty ? -1 : -2;
+    return !whole ? -2 : k < PROBE_WINDOW ? (int64_t)(s + k) : missed;
+}
+
+// Find the next slot holding `tag`, starting at `cursor` (initialise it with
+// probe_start) with `visited` slots tried, a window at a time.  Returns -1 at
+// the first empty slot or after a full cycle.  Used by join probes, which run
+// after the build kernel ended, and to go on from probe_in_window.
+template <typename Slot, typename Tag>
+DQC_DEVICE_INLINE int64_t ht_probe(const Slot* slots, uint32_t cap, Tag tag, uint32_t& cursor, uint32_t& visited) {
     while (visited < cap && visited < MAX_PROBE) {
-        const uint32_t s = cursor;
-        const uint64_t t = slots[s];
-        cursor = next_slot(s, cap);
-        ++visited;
-        if ((uint32_t)t == tag) return (int64_t)s;
-        if (t == 0ull) { visited = cap; return -1; }
+        const uint32_t s = cursor >= cap ? 0u : cursor;
+        const uint32_t rest = cap - s < cap - visited ? cap - s : cap - visited;
+        if (rest >= PROBE_WINDOW) {
+            bool empty;
+            const uint32_t k = window_find(probe_window(slots, s), tag, empty);
+            if (k < PROBE_WINDOW) {
+                cursor = s + k + 1u;
+                visited += k + 1u;
+                return (int64_t)(s + k);
+            }
+            if (empty) { visited = cap; return -1; }
+            cursor = s + PROBE_WINDOW;
+            visited += PROBE_WINDOW;
+        } else {
+            const Tag t = (Tag)slots[s];
+            cursor = s + 1u;
+            ++visited;
+            if (t == tag) return (int64_t)s;
+            if (t == (Tag)0) { visited = cap; return -1; }
+        }
     }
     return -1;
 }
@@ -544,7 +586,7 @@ DQC_DEVICE_INLINE int lds_entry(uint64_t* ltags, uint32_t nf, uint32_t rf, uint3
 // The build sets them; a probe pipeline copies the filter into LDS and skips
 // the hash-table probe of rows whose bits are not both set (no match is
 // possible), so only matches and false positives reach the table.
-DQC_DEVICE_INLINE uint32_t bloom_word(uint64_t h, uint32_t words) { return (uint32_t)h & (words - 1u); }
+DQC_DEVICE_INLINE uint32_t bloom_word(uint64_t h, uint32_t words) { return __umulhi((uint32_t)h, words); }
 DQC_DEVICE_INLINE uint32_t bloom_mask(uint64_t h) {
     return (1u << ((uint32_t)(h >> 32) & 31u)) | (1u << ((uint32_t)(h >> 40) & 31u));
 }

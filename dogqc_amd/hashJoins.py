@@ -167,7 +167,7 @@ class EquiJoinTranslator(BinaryTranslator):
                 shift += w
             pipe.emit("const uint32_t %s_key = %s;" % (hashVar, " | ".join(parts)))
             pipe.emit("%s = %s_key + 1u;" % (tagDecl, hashVar))
-            pipe.emit("const uint64_t %s = dqc::mix64(dqc::TAG_TOP | (uint64_t)%s_key);" % (hashVar, hashVar))
+            pipe.emit("const uint64_t %s = dqc::hash32(%s_key);" % (hashVar, hashVar))
         elif self.exact:
             parts = ["dqc::TAG_TOP"]
             shift = 0
@@ -305,9 +305,6 @@ class EquiJoinTranslator(BinaryTranslator):
         if ct == CType.STR_TYPE or CType.size.get(ct, 16) > 4:
             return False
         return not self._buildPartitionable(pipe)
-
-    def _probeFn(self):
-        return "dqc::ht_probe_packed" if self.packed else "dqc::ht_probe<%s>" % self.tagType
 
     def _packedWord(self, pipe, jtag):
         return "dqc::packed_slot(%s, dqc::to_word<%s>(%s))" % (jtag, self.packedType, pipe.access(self.stored[0]))
@@ -524,7 +521,7 @@ class EquiJoinTranslator(BinaryTranslator):
         with pipe.rowLoop():
             pipe.code.open("if (active[u])")
             if self.tag32:
-                pipe.emit("const uint64_t jh = dqc::mix64(dqc::TAG_TOP | (uint64_t)(%s - 1u));" % jtag)
+                pipe.emit("const uint64_t jh = dqc::hash32((uint32_t)(%s - 1u));" % jtag)
             else:
                 pipe.emit("const uint64_t jh = dqc::mix64(%s);" % jtag)
             pipe.emit("const uint32_t hs = dqc::slot_of(jh, %s);" % ins["fcap"])
@@ -799,7 +796,7 @@ class EquiJoinTranslator(BinaryTranslator):
                         pipe.code.open("else for (;;)")
                     else:
                         pipe.code.open("for (;;)")
-                    pipe.emit("%s = %s(%s, %s, %s, jcur, jv);" % (slot, self._probeFn(), ftags, fcap, jtag))
+                    pipe.emit("%s = dqc::ht_probe(%s, %s, %s, jcur, jv);" % (slot, ftags, fcap, jtag))
                     pipe.emit("if (%s < 0) break;" % slot)
                     pipe.emit("if (%s) break;" % self._matchCond(ctxt, pipe, fields, slotName))
                     pipe.code.close()
@@ -809,11 +806,9 @@ class EquiJoinTranslator(BinaryTranslator):
                     if lbf is not None:
                         pipe.code.open("if (%s)" % jf)
                     pipe.emit("uint32_t jcur = 0, jv = 0;")
-                    pipe.emit("%s = %s(%s, %s, %s, %s, jcur, jv);"
-                              % (slot, "dqc::probe_in_window_packed" if self.packed else
-                                 "dqc::probe_in_window<%s>" % tt, jw, jc, fcap, jtag))
-                    pipe.emit("if (%s == -2) %s = %s(%s, %s, %s, jcur, jv);"
-                              % (slot, slot, self._probeFn(), ftags, fcap, jtag))
+                    pipe.emit("%s = dqc::probe_in_window(%s, %s, %s, %s, jcur, jv);" % (slot, jw, jc, fcap, jtag))
+                    pipe.emit("if (%s == -2) %s = dqc::ht_probe(%s, %s, %s, jcur, jv);"
+                              % (slot, slot, ftags, fcap, jtag))
                     if self.tag32:
                         pipe.emit("if (%s == 0u) %s = %s[%s] != 0u ? (int64_t)%s : -1;"
                                   % (jtag, slot, ftags, fcap, fcap))
