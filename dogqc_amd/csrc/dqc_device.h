@@ -401,11 +401,13 @@ DQC_DEVICE_INLINE int64_t ht_probe(const Slot* slots, uint32_t cap, Tag tag, uin
 }
 
 // Group slot in exact mode: the tag is the key, so find-or-claim is one CAS
-// per probed slot with no lock.  Starts at slot s with n slots tried.
-// Returns -1 when the table is full.
-DQC_DEVICE_INLINE int64_t agg_slot_exact_from(uint64_t* tags, uint32_t cap, uint64_t tag, uint32_t s, uint32_t n,
+// per probed slot with no lock.  Probes the slots lo..hi-1 of the table from
+// slot s on, wrapping at hi (a whole table is the range 0..cap; a partitioned
+// group-by keeps each partition's groups in its own range, see part_lo).
+// Returns -1 when the range is full.
+DQC_DEVICE_INLINE int64_t agg_slot_exact_from(uint64_t* tags, uint32_t lo, uint32_t hi, uint64_t tag, uint32_t s,
                                               const uint32_t* status) {
-    for (; n < cap && n < MAX_PROBE; ++n) {
+    for (uint32_t n = 0; n < hi - lo && n < MAX_PROBE; ++n) {
         if ((n & 31u) == 31u && overflow_raised(status)) return -1;
         uint64_t t = __hip_atomic_load(&tags[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (t == tag) return (int64_t)s;
@@ -414,14 +416,28 @@ DQC_DEVICE_INLINE int64_t agg_slot_exact_from(uint64_t* tags, uint32_t cap, uint
                                       (unsigned long long)tag);
             if (prev == TAG_EMPTY || prev == tag) return (int64_t)s;
         }
-        s = next_slot(s, cap);
+        s = s + 1u == hi ? lo : s + 1u;
     }
     return -1;
 }
 
 DQC_DEVICE_INLINE int64_t agg_slot_exact(uint64_t* tags, uint32_t cap, uint64_t tag, uint64_t h,
                                          const uint32_t* status) {
-    return agg_slot_exact_from(tags, cap, tag, slot_of(h, cap), 0u, status);
+    return agg_slot_exact_from(tags, 0u, cap, tag, slot_of(h, cap), status);
+}
+
+// First slot of partition p of a partitioned group table of cap slots in
+// 2^bits partitions (bits 0: the whole table).  A key's partition is the top
+// bits of its hash and its slot a multiple of them, so a partition's home
+// slots are this range, but for a key at the range's end that rounds into the
+// next one: its home slot is the range's last (part_home).
+DQC_DEVICE_INLINE uint32_t part_of(uint64_t h, uint32_t bits) { return (uint32_t)((h >> 32) >> (32u - bits)); }
+DQC_DEVICE_INLINE uint32_t part_lo(uint32_t p, uint32_t bits, uint32_t cap) {
+    return (uint32_t)(((uint64_t)p * cap) >> bits);
+}
+DQC_DEVICE_INLINE uint32_t part_home(uint64_t h, uint32_t cap, uint32_t hi) {
+    const uint32_t s = slot_of(h, cap);
+    return s < hi ? s : hi - 1u;
 }
 
 // Key columns of a hashed group table are written by the lane that claims
@@ -531,6 +547,26 @@ DQC_DEVICE_INLINE int lds_slot_exact(uint64_t* ltags, uint32_t cap, uint64_t tag
             if (expected == tag) return (int)s;
         }
         s = next_slot(s, cap);
+    }
+    return -1;
+}
+
+// Slot of `tag` in an LDS image of n group slots, probed from slot s on and
+// wrapping at n; -1 when LDS_IMAGE_PROBE slots hold other tags.
+constexpr uint32_t LDS_IMAGE_PROBE = 512;
+
+DQC_DEVICE_INLINE int lds_image_slot(uint64_t* itags, uint32_t n, uint64_t tag, uint32_t s) {
+    for (uint32_t k = 0; k < n && k < LDS_IMAGE_PROBE; ++k) {
+        const uint64_t t = __hip_atomic_load(&itags[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (t == tag) return (int)s;
+        if (t == TAG_EMPTY) {
+            uint64_t expected = TAG_EMPTY;
+            if (__hip_atomic_compare_exchange_strong(&itags[s], &expected, tag, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                     __HIP_MEMORY_SCOPE_WORKGROUP) ||
+                expected == tag)
+                return (int)s;
+        }
+        s = s + 1u == n ? 0u : s + 1u;
     }
     return -1;
 }

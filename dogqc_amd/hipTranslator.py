@@ -551,6 +551,7 @@ class Program(object):
         h.emit("    uint32_t apbits[%d];" % max(1, len(self.hts)))
         h.emit("    int64_t apcap[%d];" % max(1, len(self.hts)))
         h.emit("    uint32_t apseg[%d];" % max(1, len(self.hts)))
+        h.emit("    uint32_t apimg[%d];" % max(1, len(self.hts)))
         h.emit("    uint32_t bfw[%d];" % max(1, len(self.hts)))
         h.emit("    uint32_t bspan[%d];" % max(1, len(self.hts)))
         h.emit("    uint32_t bspill[%d];" % max(1, len(self.hts)))
@@ -603,7 +604,7 @@ class Program(object):
             h.emit("(void)est_%d;" % opId)
         h.emit("for (int i = 0; i < %d; ++i) L.bfp[i] = 0u;" % max(1, len(self.pipes)))
         h.emit("for (int i = 0; i < %d; ++i) { L.arep[i] = 1u; L.apart[i] = 0u; L.apbits[i] = 0u; L.apcap[i] = 0; "
-               "L.apseg[i] = 0u; L.apgroups[i] = 0; L.bfw[i] = 0u; L.bspan[i] = 0u; L.bspill[i] = 0u; }"
+               "L.apseg[i] = 0u; L.apimg[i] = 0u; L.apgroups[i] = 0; L.bfw[i] = 0u; L.bspan[i] = 0u; L.bspill[i] = 0u; }"
                % max(1, len(self.hts)))
         for name, stmt in self.hostVars.items():
             # a callable is rendered now, when every pipeline is complete
@@ -820,6 +821,10 @@ def pipelineLaunch(prog, pipe, phase=None, rowsExpr=None, perCu=8):
         # one workgroup per partition; nothing to do without partitions
         lines[-1] = "const unsigned g = (unsigned)%s;" % pa["hostNp"]
         lines.append("if (g > 0u) {")
+        if "hostImg" in pa:
+            lines.append("if (%s) { kp.lw = 0u; kp.lf = 0u; }" % pa["hostImg"])
+            keep = "(uint64_t)0" if pipe.ldsFilter is None else "(uint64_t)(%s)" % pipe.ldsFilter["host"]
+            lds = "(%s ? (size_t)(%s + %s) : %s)" % (pa["hostImg"], keep, pa["hostImgBytes"], lds)
     if phase == 1 and getattr(pipe, "globalRefill", False) and pipe.ldsFilter is not None:
         # the second launch of a kernel-split lane refill runs what follows
         # the filtered probe: no filter copied into LDS, none allocated
@@ -1086,32 +1091,43 @@ def launchShape(translator):
     rows per thread: 64 M-row c0 379 us, TPC-H Q1 at SF10 268 instead of
     273 us.)"""
     U, B = rowsPerThread(translator), int(KernelCall.defaultBlockSize)
-    if pipelineShape(translator)[0] or not _fewGroupsAbove(translator):
+    groups = None if pipelineShape(translator)[0] else _groupsAbove(translator)
+    if groups is None:
         return U, B, False
     wide = min(1024, 4 * B)
-    return max(1, U * B // wide), wide, True
+    return max(1, U * B // wide), wide, groups == "few"
 
 
-def _fewGroupsAbove(translator):
-    """The pipeline ends in a group-by known to have few groups (a hint, or
-    keys of a small domain) whose keys pack into an exact tag."""
+def _groupsAbove(translator):
+    """Whether the pipeline ends in a group-by whose keys pack into an exact
+    tag and that is known to have "few" groups (a hint, or keys of a small
+    domain) or may have "many" (it can be partitioned); else None."""
+    from dogqc_amd.hashJoins import EquiJoinTranslator
     t = translator
+    joinKeys = []
     while t.parent is not None:
         p = t.parent
         if isinstance(p, BinaryTranslator) and p.leftChild is t:
-            return False
+            return None
+        if isinstance(p, EquiJoinTranslator) and not p.algExpr.multimatch:
+            joinKeys += [sorted(a.id for a in keys.values()) for keys in (p.algExpr.buildKeyAttributes,
+                                                                         p.algExpr.probeKeyAttributes)]
         if isinstance(p, AggregationTranslator):
             a = p.algExpr
             groups = list(a.groupAttributes.values()) if a.doGroup else []
             if not groups or sum(_GROUP_BITS.get(g.dataType, 65) for g in groups) > 64:
-                return False
-            if getattr(a, "numgroupsFromCfg", False):
-                return a.numgroups <= 4096
-            return _keyDomain(groups) is not None
+                return None
+            hinted = getattr(a, "numgroupsFromCfg", False)
+            if a.numgroups <= 4096 if hinted else _keyDomain(groups) is not None:
+                return "few"
+            # (a group-by on the keys of a join accumulates in that join's slots)
+            if sorted(g.id for g in groups) in joinKeys or (hinted and a.numgroups <= p.PART_MIN_GROUPS):
+                return None
+            return "many"
         if isinstance(p, MaterializeTranslator):
-            return False
+            return None
         t = p
-    return False
+    return None
 
 
 class ScanTranslator(LiteralTranslator):
@@ -1793,11 +1809,15 @@ class AggregationTranslator(UnaryTranslator):
 
     def _firstGlobalSlot(self, pipe, upd):
         gtag, gs0, gt0, ftags, fcap = upd["gtag"], upd["gs0"], upd["gt0"], upd["ftags"], upd["fcap"]
+        home = "dqc::slot_of(gh, %s)" % fcap
+        if upd.get("range"):
+            home = "dqc::part_home(gh, %s, dqc::part_lo(dqc::part_of(gh, %s) + 1u, %s, %s))" % (
+                fcap, upd["range"], upd["range"], fcap)
         if self.exact64:
-            pipe.emit("%s = %s != 0 ? dqc::slot_of(gh, %s) : %s;" % (gs0, gtag, fcap, fcap))
+            pipe.emit("%s = %s != 0 ? %s : %s;" % (gs0, gtag, home, fcap))
             pipe.emit("%s = %s != 0 ? %s[%s] : 0ull;" % (gt0, gtag, ftags, gs0))
         else:
-            pipe.emit("%s = dqc::slot_of(gh, %s);" % (gs0, fcap))
+            pipe.emit("%s = %s;" % (gs0, home))
             pipe.emit("%s = %s[%s];" % (gt0, ftags, gs0))
 
     def _globalUpdate(self, pipe, vals, upd):
@@ -1806,8 +1826,12 @@ class AggregationTranslator(UnaryTranslator):
         ftags, fcap, aoff = upd["ftags"], upd["fcap"], upd["aoff"]
         with pipe.rowLoop():
             pipe.code.open("if (%s)" % gneed)
-            pipe.emit("const int64_t gs = %s == %s ? (int64_t)%s : dqc::agg_slot_exact_from(%s, %s, %s, %s, 0u, &st->flags);"
-                      % (gt0, gtag, gs0, ftags, fcap, gtag, gs0))
+            lo, hi = "0u", fcap
+            if upd.get("range"):
+                pipe.emit("const uint32_t gpart = dqc::part_of(dqc::mix64(%s), %s);" % (gtag, upd["range"]))
+                lo, hi = ["dqc::part_lo(gpart%s, %s, %s)" % (x, upd["range"], fcap) for x in ("", " + 1u")]
+            pipe.emit("const int64_t gs = %s == %s ? (int64_t)%s : dqc::agg_slot_exact_from(%s, %s, %s, %s, %s, &st->flags);"
+                      % (gt0, gtag, gs0, ftags, lo, hi, gtag, gs0))
             pipe.code.open("if (gs >= 0)")
             for acc, v in zip(self.accs, vals):
                 pipe.emit(_guarded(acc, "%s;" % _atomic(acc["kind"], "%s[%s + gs]" % (acc["field"], aoff), v)))
@@ -1823,12 +1847,15 @@ class AggregationTranslator(UnaryTranslator):
 
     # partitioned group-by: at most this many partitions and first-pass
     # workgroups (segments per partition); auto mode above this many groups
-    # (below, the LDS table holds a workgroup's groups), aiming at this many
-    # groups per partition
+    # (below, the LDS table holds a workgroup's groups) and rows (the second
+    # launch costs 5 us), aiming at this many groups per partition and at
+    # least a workgroup per CU
     PART_MAX = 1024
     PART_SEG_MAX = 2048
-    PART_MIN_GROUPS = 16384
+    PART_MIN_GROUPS = 2048
+    PART_MIN_ROWS = 65536
     PART_GROUPS = 256
+    PART_AUTO_MIN = 256
 
     def _partitionable(self, pipe):
         """A group-by with many groups updates the global table once per row,
@@ -1859,13 +1886,29 @@ class AggregationTranslator(UnaryTranslator):
         in the loop; rows that do not fit their segment (and the tag-0 key)
         update the global table directly.  At its end the workgroup stores
         its segment counts.  PHASE 1 gives workgroup b partition b: its rows
-        are the records of the segments of partition b, aggregated in the
-        LDS table (slots from the hash bits below the partition bits) and
-        flushed once per group.  Partitions hold disjoint groups, so the
-        global table receives one update per group and workgroup instead of
-        one per row.  With no partitions (tuning part_agg, or a small or
-        unknown group count) PHASE 0 is the plain exact-tag update and
-        PHASE 1 is not launched."""
+        are the records of the segments of partition b.  The top bits that
+        pick a row's partition also pick its home slot, so a partition's
+        groups have a range of the group table's slots to themselves
+        (dqc::part_lo).  The workgroup holds that range in LDS (the image),
+        aggregates there and writes the used slots back with plain stores:
+        no claim and no atomic leaves the CU.  What PHASE 0 put into the
+        range directly is read into the image first.  Every update of such a
+        table wraps its probes inside the range, and a full range reports an
+        overflow like a full table.  A range too large for LDS (beyond about
+        8 M groups of one accumulator) is aggregated in an LDS table instead
+        and flushed group by group, with slots over the whole table.
+
+        Flushing every group with a claim and an atomic per accumulator took
+        277 us for 1.5 M groups of 6 M rows and 94 us for 106 k groups of
+        3.2 M rows; the image takes 68 and 64 us (with 1024 threads a
+        workgroup; with 256, too few wavefronts for the records' latency, 135
+        and 116).  At 8 k groups of 246 k rows, 70 us unpartitioned, 25 us
+        partitioned; 16 k of 1.1 M, 172 and 58.  Fewer than one partition per
+        CU leaves CUs idle (64 partitions: 25 us in the second launch alone).
+
+        With no partitions (tuning part_agg, or a small or unknown group
+        count) PHASE 0 is the plain exact-tag update and PHASE 1 is not
+        launched."""
         a = self.algExpr
         G = a.opId
         idx = self.ht["index"]
@@ -1874,13 +1917,19 @@ class AggregationTranslator(UnaryTranslator):
         cfgParts = 0
         if getattr(a, "partitions", None):
             cfgParts = min(self.PART_MAX, max(2, _pow2floor(int(a.partitions))))
+        slotBytes = 8 + sum(CType.size[acc["ctype"]] for acc in self.accs)
+
+        def used():
+            # LDS beside the image: static arrays (the three below among them), a join filter in front
+            f = "" if pipe.ldsFilter is None else " + " + pipe.ldsFilter["host"]
+            return "(uint64_t)%du%s" % (staticLdsBytes(pipe) + 4 * (self.PART_MAX + self.PART_SEG_MAX + 1 + 17) + 1024, f)
         prog.hostVars["apart%d" % idx] = (
             "{ const int32_t req = t->part_agg;\n"
             "  const int64_t known = t->ht_capacity[%d] > 0 ? t->ht_capacity[%d] / 2 : %s;\n"
             "  uint32_t np = 0u;\n"
             "  if (req > 0) np = std::min<uint32_t>(%du, std::max<uint32_t>(2u, pow2floor((uint64_t)req)));\n"
             "  else if (req == 0 && %d > 0) np = %du;\n"
-            "  else if (req == 0 && known > %d) np = std::min<uint32_t>(%du, std::max<uint32_t>(2u, pow2ceil((uint64_t)(known / %d))));\n"
+            "  else if (req == 0 && known > %d && %s >= %d) np = std::min<uint32_t>(%du, std::max<uint32_t>(%du, pow2ceil((uint64_t)(known / %d))));\n"
             "  uint32_t bits = 0u; while ((1u << bits) < np) ++bits;\n"
             "  L.apart[%d] = np; L.apbits[%d] = bits;\n"
             "  L.apgroups[%d] = known > 0 ? known : %s;\n"
@@ -1889,12 +1938,14 @@ class AggregationTranslator(UnaryTranslator):
             "    const double mu = (double)std::max<int64_t>(1, %s) / ((double)seg * np);\n"
             "    L.apseg[%d] = seg;\n"
             "    L.apcap[%d] = std::min<int64_t>(((int64_t)1 << 31) / seg, (int64_t)(mu * 1.25 + 4.0 * std::sqrt(mu)) + 16);\n"
+            "    const uint64_t span = (uint64_t)L.htcap[%d] / np + 1u;\n"
+            "    L.apimg[%d] = L.htcap[%d] >= (int64_t)np && span * %du + 256u + %s <= maxLds() ? (uint32_t)span : 0u;\n"
             "  } }"
-            % (idx, idx, groupsKnown, self.PART_MAX, cfgParts, cfgParts, self.PART_MIN_GROUPS, self.PART_MAX,
-               self.PART_GROUPS,
+            % (idx, idx, groupsKnown, self.PART_MAX, cfgParts, cfgParts, self.PART_MIN_GROUPS,
+               prog.estimate(a.child), self.PART_MIN_ROWS, self.PART_MAX, self.PART_AUTO_MIN, self.PART_GROUPS,
                idx, idx, idx, est,
                self.PART_SEG_MAX, pipe.pipeId, pipe.pipeId, pipe.defaultGrid, pipe.params["n"][1], B * U,
-               prog.estimate(a.child), idx, idx))
+               prog.estimate(a.child), idx, idx, idx, idx, idx, slotBytes, used()))
         # a record is 1 + (inputs) 8-byte words, stored row-wise so that a
         # partition's records in a segment share cache lines
         K = 1 + sum(1 for acc in self.accs if acc["kind"] != "count")
@@ -1903,6 +1954,11 @@ class AggregationTranslator(UnaryTranslator):
         fbits = pipe.param("pbits%d" % G, "uint32_t", "L.apbits[%d]" % idx)
         fseg = pipe.param("pseg%d" % G, "uint32_t", "L.apseg[%d]" % idx)
         fpcap = pipe.param("pcap%d" % G, "uint32_t", "L.apcap[%d]" % idx)
+        fimg = pipe.param("pimg%d" % G, "uint32_t", "L.apimg[%d]" % idx)
+        # partitions as ranges of table slots, with the image (else one range)
+        upd["range"] = pipe.param("prb%d" % G, "uint32_t", "L.apimg[%d] ? L.apbits[%d] : 0u" % (idx, idx))
+        bdir = prog.buffer("apd%d" % G, CType.UINT, "(uint64_t)L.apart[%d]" % idx, "0x0ull")
+        fdir = pipe.param("apd%d" % G, "uint32_t*", "B_" + bdir)
         bcnt = prog.buffer("apc%d" % G, CType.UINT, "(uint64_t)L.apart[%d] * L.apseg[%d]" % (idx, idx))
         fcnt = pipe.param("apc%d" % G, "uint32_t*", "B_" + bcnt)
         brec = prog.buffer("aprec%d" % G, CType.UINT64, recs)
@@ -1947,6 +2003,7 @@ class AggregationTranslator(UnaryTranslator):
             pipe.code.open("else")
             pipe.emit("// segment full, or the tag-0 key: the global table")
             pipe.emit("%s = 1;" % gneed)
+            pipe.emit("%s[pb] = 1u;" % fdir)
             self._firstGlobalSlot(pipe, upd)
             pipe.code.close()
             pipe.code.close()
@@ -1971,8 +2028,55 @@ class AggregationTranslator(UnaryTranslator):
         vals1 = []
         for acc, v in zip(self.accs, vals):
             vals1.append(v if acc["i"] not in words else "dqc::from_word<%s>(%s)" % (acc["ctype"], pvals[acc["i"]]))
-        self._exactUpdate(pipe, ptag, vals1, upd, "(gh << %s)" % fbits)
+        pipe.code.open("if (%s == 0u)" % fimg)
+        self._exactUpdate(pipe, ptag, vals1, dict(upd, range=None), "(gh << %s)" % fbits)
         pipe.code.close()
+        pipe.code.open("else")
+        with pipe.rowLoop():
+            pipe.code.open("if (active[u])")
+            pipe.emit("const uint64_t gh = dqc::mix64(%s);" % ptag)
+            pipe.emit("const int li = dqc::lds_image_slot(itags, ihi - ilo, %s, dqc::part_home(gh, %s, ihi) - ilo);"
+                      % (ptag, upd["fcap"]))
+            pipe.code.open("if (li >= 0)")
+            for acc, v in zip(self.accs, vals1):
+                pipe.emit(_ldsOp(acc["kind"], "&iacc%d[li]" % acc["i"], v))
+            pipe.code.close()
+            pipe.emit(upd["overflow"])
+            pipe.code.close()
+        pipe.code.close()
+        pipe.code.close()
+        # the image: this partition's slots of the group table, in LDS; what
+        # PHASE 0 put there directly (seldom anything) is read in first
+        pro, ep = pipe.prologue, pipe.epilogue
+        base = "0u" if pipe.ldsFilter is None else pipe.ldsFilter["dev"]
+        pro.emit("uint64_t* itags = (uint64_t*)(dqc_dyn_lds + %s);" % base)
+        pro.emit("uint64_t ioff = %s + (uint64_t)%s * 8u;" % (base, fimg))
+        for acc in self.accs:
+            pro.emit("%s* iacc%d = (%s*)(dqc_dyn_lds + ioff);" % (acc["ctype"], acc["i"], acc["ctype"]))
+            pro.emit("ioff += ((uint64_t)%s * %d + 7u) & ~(uint64_t)7u;" % (fimg, CType.size[acc["ctype"]]))
+        pro.emit("uint32_t ilo = 0u, ihi = 0u;")
+        pro.open("if (PHASE == 1 && %s > 0u && blockIdx.x < %s)" % (fimg, fnp))
+        pro.emit("ilo = dqc::part_lo(blockIdx.x, %s, %s); ihi = dqc::part_lo(blockIdx.x + 1u, %s, %s);"
+                 % (fbits, upd["fcap"], fbits, upd["fcap"]))
+        pro.emit("const bool before = %s[blockIdx.x] != 0u;" % fdir)
+        pro.open("for (uint32_t i = threadIdx.x; i < ihi - ilo; i += %du)" % B)
+        pro.emit("itags[i] = before ? %s[ilo + i] : 0ull;" % upd["ftags"])
+        for acc in self.accs:
+            pro.emit("iacc%d[i] = before ? %s[%s + ilo + i] : %s;" % (acc["i"], acc["field"], upd["aoff"],
+                                                                      _cIdentity(acc["kind"], acc["ctype"])))
+        pro.close()
+        pro.emit("__syncthreads();")
+        pro.close()
+        ep.open("if (PHASE == 1 && ihi > ilo)")
+        ep.emit("__syncthreads();")
+        ep.open("for (uint32_t i = threadIdx.x; i < ihi - ilo; i += %du)" % B)
+        ep.open("if (itags[i] != 0ull)")
+        ep.emit("%s[ilo + i] = itags[i];" % upd["ftags"])
+        for acc in self.accs:
+            ep.emit("%s[%s + ilo + i] = iacc%d[i];" % (acc["field"], upd["aoff"], acc["i"]))
+        ep.close()
+        ep.close()
+        ep.close()
         # PHASE 0 end: the segment counts
         pipe.epilogue.open("if (PHASE == 0 && %s > 0u)" % fnp)
         pipe.epilogue.emit("__syncthreads();")
@@ -1982,8 +2086,12 @@ class AggregationTranslator(UnaryTranslator):
         pipe.phased = True
         pipe.phaseBetween = []
         pipe.partAgg = {"np": fnp, "cap": fpcap, "count": fcnt, "nseg": fseg, "pref": pref, "scan": scan,
-                        "hostNp": "L.apart[%d]" % idx, "hostNseg": "L.apseg[%d]" % idx}
-        # the LDS table of PHASE 1: sized for 4x the groups of one partition
+                        "hostNp": "L.apart[%d]" % idx, "hostNseg": "L.apseg[%d]" % idx,
+                        "hostImg": "L.apimg[%d]" % idx,
+                        "hostImgBytes": " + ".join(["(uint64_t)L.apimg[%d] * 8u" % idx] + [
+                            "(((uint64_t)L.apimg[%d] * %d + 7u) & ~(uint64_t)7u)" % (idx, CType.size[acc["ctype"]])
+                            for acc in self.accs])}
+        # the LDS table of PHASE 1 (without the image): sized for 4x the groups of one partition
         # (short probes; measured on 234 groups per partition: 2048 slots
         # 89 us, 512 slots 110 us), at most 4096 slots
         return ("(L.apart[%d] ? std::min<int64_t>(2048, std::max<int64_t>(1, 4 * L.apgroups[%d] / (int64_t)L.apart[%d])) : %s)"
