@@ -15,10 +15,14 @@
 #include <unistd.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
 #include <string>
+#include <unordered_map>
+#include <vector>
 
 #include "dogqc_amd.h"
 #include "dqc_runtime_internal.h"
@@ -84,6 +88,111 @@ bool adjustForRetry(const dqc_plan_layout& L, const dqc_plan_status& st, dqc_pla
     return retry;
 }
 
+namespace {
+
+constexpr uint64_t WS_KEEP_BYTES = 2ull << 30;
+constexpr size_t WS_KEEP_BLOCKS = 16;
+constexpr uint64_t WS_KEEP_ACQUIRES = 256;
+
+struct WsBlock {
+    void* ptr;
+    uint64_t bytes;
+    int device;
+    uint64_t since;     // acquisitions so far when it was released
+};
+
+struct WsPool {
+    std::mutex lock;
+    std::vector<WsBlock> free;                      // oldest release first
+    std::unordered_map<void*, WsBlock> out;         // handed out
+    uint64_t acquires = 0;
+};
+
+// (never destroyed: nothing is freed after the HIP runtime's own end)
+WsPool& pool() {
+    static WsPool* p = new WsPool();
+    return *p;
+}
+
+std::atomic<int> g_modules{0};
+
+}  // namespace
+
+void wsTrim() {
+    std::vector<WsBlock> all;
+    {
+        std::lock_guard<std::mutex> g(pool().lock);
+        all.swap(pool().free);
+    }
+    for (const WsBlock& b : all) (void)hipFree(b.ptr);
+}
+
+int wsAcquire(void** ptr, uint64_t bytes) {
+    *ptr = nullptr;
+    if (bytes == 0) bytes = 256;
+    int device = 0;
+    HIP_CHECK(hipGetDevice(&device), "hipGetDevice");
+    WsPool& p = pool();
+    {
+        std::lock_guard<std::mutex> g(p.lock);
+        ++p.acquires;
+        size_t best = p.free.size();
+        for (size_t i = 0; i < p.free.size(); ++i)
+            if (p.free[i].device == device && p.free[i].bytes >= bytes &&
+                (best == p.free.size() || p.free[i].bytes < p.free[best].bytes))
+                best = i;
+        if (best < p.free.size()) {
+            const WsBlock b = p.free[best];
+            p.free.erase(p.free.begin() + (long)best);
+            p.out[b.ptr] = b;
+            *ptr = b.ptr;
+            return DQC_OK;
+        }
+    }
+    const int rc = dqc_malloc(ptr, bytes);
+    if (rc) return rc;
+    std::lock_guard<std::mutex> g(p.lock);
+    p.out[*ptr] = WsBlock{*ptr, bytes, device, 0};
+    return DQC_OK;
+}
+
+int wsRelease(void* ptr) {
+    if (!ptr) return DQC_OK;
+    WsPool& p = pool();
+    WsBlock b{nullptr, 0, -1, 0};
+    {
+        std::lock_guard<std::mutex> g(p.lock);
+        const auto it = p.out.find(ptr);
+        if (it != p.out.end()) {
+            b = it->second;
+            p.out.erase(it);
+        }
+    }
+    int device = -1;
+    if (!b.ptr || b.bytes > WS_KEEP_BYTES || hipGetDevice(&device) != hipSuccess || device != b.device ||
+        hipDeviceSynchronize() != hipSuccess) {
+        (void)hipGetLastError();
+        HIP_CHECK(hipFree(ptr), "hipFree");
+        return DQC_OK;
+    }
+    std::vector<void*> drop;
+    {
+        std::lock_guard<std::mutex> g(p.lock);
+        b.since = p.acquires;
+        p.free.push_back(b);
+        uint64_t kept = 0;
+        for (const WsBlock& f : p.free) kept += f.bytes;
+        while (kept > WS_KEEP_BYTES || p.free.size() > WS_KEEP_BLOCKS ||
+               p.acquires - p.free.front().since > WS_KEEP_ACQUIRES) {
+            kept -= p.free.front().bytes;
+            drop.push_back(p.free.front().ptr);
+            p.free.erase(p.free.begin());
+        }
+    }
+    for (void* d : drop) (void)hipFree(d);
+    return DQC_OK;
+}
+
 }  // namespace dqcrt
 
 extern "C" {
@@ -109,6 +218,11 @@ int dqc_malloc(void** ptr, uint64_t bytes) {
     *ptr = nullptr;
     if (bytes == 0) bytes = 256;
     hipError_t e = hipMalloc(ptr, bytes);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        dqcrt::wsTrim();
+        e = hipMalloc(ptr, bytes);
+    }
     if (e != hipSuccess) {
         (void)hipGetLastError();
         return fail(DQC_ENOMEM, "hipMalloc(%llu): %s", (unsigned long long)bytes, hipGetErrorString(e));
@@ -221,6 +335,7 @@ int dqc_module_load(const char* so_path, void** module) {
         delete m;
         return fail(DQC_ELOAD, "%s does not export the dqc_plan ABI", so_path);
     }
+    ++dqcrt::g_modules;
     *module = m;
     return DQC_OK;
 }
@@ -230,6 +345,7 @@ int dqc_module_unload(void* module) {
     if (!m) return DQC_OK;
     dlclose(m->handle);
     delete m;
+    if (--dqcrt::g_modules == 0) dqcrt::wsTrim();
     return DQC_OK;
 }
 
@@ -260,9 +376,10 @@ int dqc_query_run(void* module, const dqc_plan_inputs* in, dqc_plan_tuning* tun,
         int rc = m->layout(in, tun, &L);
         if (rc) return fail(rc, "plan layout failed (%d)", rc);
         if (res->ws == nullptr || res->ws_bytes < L.ws_bytes) {
-            if (res->ws) dqc_free(res->ws);
+            void* old = res->ws;
             res->ws = nullptr;
-            rc = dqc_malloc(&res->ws, L.ws_bytes);
+            if (old && (rc = dqcrt::wsRelease(old)) != DQC_OK) return rc;
+            rc = dqcrt::wsAcquire(&res->ws, L.ws_bytes);
             if (rc) return rc;
             res->ws_bytes = L.ws_bytes;
         }
@@ -283,7 +400,7 @@ int dqc_query_run(void* module, const dqc_plan_inputs* in, dqc_plan_tuning* tun,
 
 int dqc_query_release(dqc_query_result* res) {
     if (!res) return DQC_OK;
-    int rc = dqc_free(res->ws);
+    int rc = dqcrt::wsRelease(res->ws);
     res->ws = nullptr;
     res->ws_bytes = 0;
     return rc;

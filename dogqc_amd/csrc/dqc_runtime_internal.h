@@ -25,6 +25,25 @@ struct Module {
 // their exact counts).  Returns true when the run has to be repeated.
 bool adjustForRetry(const dqc_plan_layout& L, const dqc_plan_status& st, dqc_plan_tuning* tun);
 
+// Workspaces of dqc_query_run.  A workspace handed out is an allocation of
+// its own (hipMalloc); one that is released waits here for the next run that
+// fits it, because allocating and freeing costs more than most plans: 0.3 ms
+// for 100 MB and more, and 8 ms where the process holds gigabytes (a TPC-H Q18
+// call at SF1 9.0 ms, 0.34 ms with waiting workspaces).
+//   * bounded: at most 2 GiB and 16 blocks wait, the oldest are freed first;
+//     a larger workspace is freed at once;
+//   * given back: blocks no run has asked for in 256 acquisitions are freed,
+//     all when an allocation of this library fails and when the last plan
+//     module is unloaded;
+//   * released like hipFree: the device's pending work is waited for, so work
+//     on any stream that still reads the results has ended before the memory
+//     is handed out again;
+//   * safe with several threads (a lock around the list) and devices (a block
+//     goes only to runs on its own device).
+int wsAcquire(void** ptr, uint64_t bytes);
+int wsRelease(void* ptr);
+void wsTrim();
+
 }  // namespace dqcrt
 
 #define HIP_CHECK(expr, what)                                      \

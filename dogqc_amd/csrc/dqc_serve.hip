@@ -563,6 +563,11 @@ int dqc_serve_create(const dqc_serve_config* cfg, void** server) {
     hipError_t e = hipMalloc(&base, cfg->arena_bytes);
     if (e != hipSuccess) {
         (void)hipGetLastError();
+        dqcrt::wsTrim();
+        e = hipMalloc(&base, cfg->arena_bytes);
+    }
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
         return fail(DQC_ENOMEM, "arena of %llu bytes: %s", (unsigned long long)cfg->arena_bytes,
                     hipGetErrorString(e));
     }

@@ -337,13 +337,26 @@ class Execution(object):
     def count(self):
         return int(self.res.status.result_count)
 
+    # a result whose columns lie this close together is copied at once: a copy
+    # to the host takes 17 us however small (c0's result, ten columns of six
+    # rows: 25 us at once)
+    ONE_COPY_BYTES = 65536
+
     def columns(self):
         """Result columns as an OrderedDict name -> numpy array."""
         out = OrderedDict()
         n = min(self.count, int(self.res.layout.result_capacity))
-        for i, c in enumerate(self.module.desc["result"]):
-            dt = CTYPE_DTYPE[c["ctype"]]
-            out[c["name"]] = copyToHost(self.res.ws + self.res.layout.result_offset[i], dt, n)
+        cols = [(c["name"], CTYPE_DTYPE[c["ctype"]], int(self.res.layout.result_offset[i]))
+                for i, c in enumerate(self.module.desc["result"])]
+        lo = min((off for _, _, off in cols), default=0)
+        span = max((off + n * np.dtype(dt).itemsize for _, dt, off in cols), default=0) - lo
+        if n and span <= self.ONE_COPY_BYTES:
+            raw = copyToHost(self.res.ws + lo, np.uint8, span)
+            for name, dt, off in cols:
+                out[name] = raw[off - lo:off - lo + n * np.dtype(dt).itemsize].view(dt).copy()
+            return out
+        for name, dt, off in cols:
+            out[name] = copyToHost(self.res.ws + off, dt, n)
         return out
 
     def tempCount(self, name):
