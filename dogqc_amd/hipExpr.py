@@ -167,10 +167,8 @@ def likeMatcherDecl(name, pattern, lit):
         H = min(len(b), 8)
         head = 0
         for k in range(H):
-            head = (head << 8) | b[k]
-        hmask = (1 << (8 * H)) - 1
-        body.append("    pos = dqc::string_find(pos, lim, %s, %du, 0x%xull, 0x%xull, %du);"
-                    % (lit(m)[1], len(b), head, hmask, H))
+            head |= b[k] << (8 * k)
+        body.append("    pos = dqc::string_find<%du>(pos, lim, %s, %du, 0x%xull);" % (H, lit(m)[1], len(b), head))
         body.append("    if (!pos) return false;")
     body.append("    return true;")
     body.append("}")
