@@ -158,6 +158,7 @@ class Pipeline(object):
         self.refillPoints = []
         self.annotations = []
         self.fewGroups = False       # ends in a group-by known to have few groups (launchShape)
+        self.rankedRows = False      # the second launch reads which rows passed the filters
         self.sharedAtomics = False   # every workgroup updates the same few words
         self.innerDepth = 0
         self.probedJoins = []
@@ -1178,7 +1179,36 @@ class ScanTranslator(LiteralTranslator):
         pipe.param("st", "dqc_plan_status*", "st")
         self._finish(ctxt, pipe)
 
+    def _rankedRows(self):
+        """Whether the pipeline only filters and maps on its way into a
+        multimap build, with a filter on strings: then the first launch's
+        rank per row (EquiJoinTranslator._multiBuildStaged), written for
+        every row, tells the second which rows to insert, instead of the
+        filter once more.  (For other filters the second launch reads about
+        as many bytes either way, and the first would write more.)"""
+        from dogqc_amd.hashJoins import EquiJoinTranslator
+        t, strings = self, False
+        while t.parent is not None:
+            p = t.parent
+            if isinstance(p, EquiJoinTranslator):
+                return p if strings and p.leftChild is t and p.algExpr.multimatch else None
+            if isinstance(p, SelectionTranslator):
+                strings = strings or any(a.dataType == Type.STRING for a in p.algExpr.conditionAttributes.values())
+            elif not isinstance(p, (MapTranslator, ProjectionTranslator)):
+                return None
+            t = p
+        return None
+
     def _finish(self, ctxt, pipe):
+        build = self._rankedRows()
+        if build is not None:
+            J = build.algExpr.opId
+            pipe.rankedRows = True
+            f = pipe.param("mmr%d" % J, "uint32_t*", "B_mmr%d" % J)
+            pipe.code.open("if constexpr (PHASE == 1)")
+            with pipe.rowLoop():
+                pipe.emit("if (active[u]) active[u] = %s[%s[u]] != 0xffffffffu;" % (f, pipe.tid))
+            pipe.code.close()
         fracs = firstUseFractions(self)
         eager = []
         for id, attr in self.algExpr.outRelation.items():
@@ -1277,8 +1307,14 @@ class SelectionTranslator(UnaryTranslator):
         pipe.emit("// selection (opId %d)" % self.algExpr.opId)
         pipe.need(self.algExpr.conditionAttributes.values())
         cond = ctxt.exprEmitter().emit(self.algExpr.condition)
+        if pipe.rankedRows:
+            # the second launch knows the rows that passed (columns that only
+            # the condition reads are then dead loads, which the compiler drops)
+            pipe.code.open("if constexpr (PHASE == 0)")
         with pipe.rowLoop():
             pipe.emit("if (active[u]) active[u] = (%s) ? 1 : 0;" % cond)
+        if pipe.rankedRows:
+            pipe.code.close()
         self.parent.consume(ctxt)
 
 

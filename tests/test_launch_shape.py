@@ -69,3 +69,19 @@ def test_front_table(groups, n):
     acc.data[("t", "t_grp")] = (np.arange(n) % groups - 1).astype(np.int32)
     check("f_groupby_64", acc, label="groups=%d n=%d" % (groups, n))
     check("f_groupby_wide", acc, label="groups=%d n=%d" % (groups, n))
+
+
+# a string filter into a multimap build: the second launch takes the rows
+# that passed from the first launch's ranks, tiled and in steps of the grid
+@pytest.mark.gpu
+@pytest.mark.parametrize("orders", [8, 255, 3071, 3072, 3073])
+@pytest.mark.parametrize("grid", [0, GRID])
+def test_ranked_rows(orders, grid):
+    from dogqc_amd import tpch
+    from dogqc_amd.dbio import MemoryAccessor
+    acc = MemoryAccessor(tpch.generate(orders / 1.5e6, seed=orders))
+    t = rt.newTuning()
+    for i in range(rt.MAX_PIPES):
+        t.grid[i] = grid
+    for q in ("tpch13", "tpch16"):
+        check(q, acc, tuning=t, label="orders=%d" % orders)
