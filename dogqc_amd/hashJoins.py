@@ -949,6 +949,10 @@ class EquiJoinTranslator(BinaryTranslator):
         else:
             pipe.code.open("while (dqc::ballot(mact%d))" % J)
             pipe.emit("%s = %s;" % (pos, moff))
+        outerLoop = pipe.loopInvariant
+        # (a loop nested in a lane-reassigning one is left alone)
+        pipe.loopInvariant = set(id for id, st in pipe.attrs.items() if st.loaded) if pipe.innerDepth == 0 else None
+        exits, pipe.loopExit = pipe.loopExit, []
         self._bindBuild(pipe, fields, posName, nullReg)
         pipe.emit("active[u] = mact%d;" % J)
         pipe.emit("if (active[u]) active[u] = (%s) ? 1 : 0;" % self._matchCond(ctxt, pipe, fields, posName,
@@ -964,6 +968,9 @@ class EquiJoinTranslator(BinaryTranslator):
         pipe.emit("++%s;" % moff)
         pipe.emit("mact%d = mact%d && %s < %s;" % (J, J, moff, mend))
         pipe.code.close()
+        for emit in pipe.loopExit:
+            emit()
+        pipe.loopInvariant, pipe.loopExit = outerLoop, exits
         pipe.emit("active[u] = 0;")
 
     def _splitEnabled(self, pipe):

@@ -162,6 +162,8 @@ class Pipeline(object):
         self.sharedAtomics = False   # every workgroup updates the same few words
         self.innerDepth = 0
         self.probedJoins = []
+        self.loopInvariant = None   # attribute ids loaded before the per-lane match loop being emitted
+        self.loopExit = []          # emitters to run after that loop, with its rows' lanes as they are
         self.nullFlags = {}         # attribute id -> null flag (outer-join build attributes)
         self.loopOps = 0            # operators so far that reassign tuples to lanes
         self.uniqueCount = 0
@@ -1771,6 +1773,62 @@ class AggregationTranslator(UnaryTranslator):
                     % (1 << idx))
 
         self.keyBuffers = []
+        if self._perProbeRow(pipe, groups):
+            vals = self._accumulateOverLoop(pipe, vals)
+            # (the null flags were honoured there; the update is emitted below
+            # the loop, when the probe row's lane is done with its matches)
+            for acc in self.accs:
+                acc["null"] = None
+            pipe.loopExit.append(lambda: self._emitUpdate(ctxt, pipe, prog, groups, packed, vals, ftags, fcap, aoff,
+                                                          est, overflow, arepVar, loopHit="ghit%d" % a.opId))
+            if not self.exact:
+                self._keyColumns(pipe, prog, groups)
+            return
+        self._emitUpdate(ctxt, pipe, prog, groups, packed, vals, ftags, fcap, aoff, est, overflow, arepVar)
+
+    def _perProbeRow(self, pipe, groups):
+        """The group-by sits in a per-lane match loop and its keys are values
+        of the probe row: every match of a row goes to the same group."""
+        return pipe.loopInvariant is not None and pipe.innerDepth == 1 and \
+            all(g.id in pipe.loopInvariant for g in groups)
+
+    def _accumulateOverLoop(self, pipe, vals):
+        """Accumulate a probe row's matches in registers, so that the row
+        updates its group once, after the match loop, instead of once per
+        match (TPC-H Q13, 1.5 M matches of 100 k customers: 212 -> 51 us).
+        Returns the registers as the update's values."""
+        G = self.algExpr.opId
+        hit = pipe.reg("ghit%d" % G, "int", "0", perRow=False)
+        regs = []
+        for acc in self.accs:
+            regs.append(pipe.reg("gacc%d_%d" % (G, acc["i"]), acc["ctype"], _cIdentity(acc["kind"], acc["ctype"]),
+                                 perRow=False))
+        pipe.code.open("if (active[u])")
+        pipe.emit("%s = 1;" % hit)
+        for acc, r, v in zip(self.accs, regs, vals):
+            pipe.emit(_guarded(acc, _combine(acc["kind"], r, v)))
+        pipe.code.close()
+        return regs
+
+    def _keyColumns(self, pipe, prog, groups):
+        """Key columns of a hashed group table."""
+        a = self.algExpr
+        idx = self.ht["index"]
+        self.keyFields = []
+        for k, g in enumerate(groups):
+            ct = pipe.attrs[g.id].ctype
+            b = prog.buffer("aht%d_k%d" % (a.opId, k), ct, "L.htcap[%d]" % idx)
+            self.keyBuffers.append((b, ct))
+            self.keyFields.append(pipe.param("aht%d_k%d" % (a.opId, k), "%s*" % ct, "B_" + b))
+
+    def _emitUpdate(self, ctxt, pipe, prog, groups, packed, vals, ftags, fcap, aoff, est, overflow, arepVar,
+                    loopHit=None):
+        """The group update of the active rows; with loopHit, of the rows
+        that matched in the loop just closed, whose accumulator registers
+        are reset for the next ones."""
+        a = self.algExpr
+        if loopHit is not None:
+            pipe.emit("active[u] = %s;" % loopHit)
         if self.exact:
             tagExpr, self.unpack, _ = packed
             G = a.opId
@@ -1785,13 +1843,9 @@ class AggregationTranslator(UnaryTranslator):
                 self._ldsTier(ctxt, pipe, prog, ftags, fcap, est, aoff)
             arepVar()
         else:
-            keyFields = []
-            for k, g in enumerate(groups):
-                ct = pipe.attrs[g.id].ctype
-                b = prog.buffer("aht%d_k%d" % (a.opId, k), ct, "L.htcap[%d]" % idx)
-                self.keyBuffers.append((b, ct))
-                keyFields.append(pipe.param("aht%d_k%d" % (a.opId, k), "%s*" % ct, "B_" + b))
-            self.keyFields = keyFields
+            if not self.keyBuffers:
+                self._keyColumns(pipe, prog, groups)
+            keyFields = self.keyFields
             with pipe.rowLoop():
                 pre = hoistStringHashes(pipe, groups)
                 pipe.code.open("if (active[u])")
@@ -1814,6 +1868,10 @@ class AggregationTranslator(UnaryTranslator):
                 pipe.emit(overflow)
                 pipe.code.close()
             arepVar()
+        if loopHit is not None:
+            pipe.emit("%s = 0;" % loopHit)
+            for acc, r in zip(self.accs, vals):
+                pipe.emit("%s = %s;" % (r, _cIdentity(acc["kind"], acc["ctype"])))
 
     def _exactUpdate(self, pipe, tagCode, vals, upd, ldsHash):
         """Exact-tag group update of the active rows: the LDS table when the
