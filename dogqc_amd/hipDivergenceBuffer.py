@@ -10,8 +10,8 @@ inner loops are skipped (cudaDivergenceBuffer.py:21-24).
 Two buffer kinds, selected like the reference's BufferType
 (cudaDivergenceBuffer.py:44-46) through ``LaneRefill.bufferType``:
 
-* ``BufferType.SMEM`` (default): every wavefront owns a 128-entry LDS queue
-  per live register (attributes already in registers, plus the row indices
+* ``BufferType.SMEM`` (default): every wavefront owns an LDS queue per live
+  register (64 entries and 64 more per row that a thread carries up to here) (attributes already in registers, plus the row indices
   of attributes that are still loaded lazily, so columns that only later
   operators read are fetched after compaction, for dense lanes only).
   Survivors are appended with one 64-bit ballot and an mbcnt prefix; the
@@ -77,15 +77,28 @@ class LaneRefill(UnaryTranslator):
         return self.algExpr.opId + 100000
 
     def consume(self, ctxt):
+        self.refill(ctxt, list(self.algExpr.outRelation.values()), self.parent.consume)
+
+    def possible(self, ctxt):
+        """Whether rows can be reassigned to lanes here: not inside an inner
+        loop, and several rows per thread only into an LDS queue."""
+        pipe = ctxt.pipe
+        return not (ctxt.innerLoopCount > 0 or pipe.innerDepth > 0 or
+                    (pipe.U != 1 and self.bufferType is not BufferType.SMEM))
+
+    def refill(self, ctxt, attrs, above):
+        """Park the active rows with the given attributes; `above` emits the
+        operators that run on the released ones."""
         pipe = ctxt.pipe
         X = self.algExpr.opId
-        if ctxt.innerLoopCount > 0 or pipe.innerDepth > 0 or pipe.U != 1:
+        if not self.possible(ctxt):
             pipe.emit("// lane refill at opId %d skipped inside an inner loop" % X)
-            self.parent.consume(ctxt)
+            above(ctxt)
             return
+        self.above = above
         pipe.annotations.append("LR%d" % X)
         pipe.loopOps += 1
-        live = pipe.liveState(self.algExpr.outRelation.values())
+        live = pipe.liveState(attrs)
         if pipe.tid not in live:
             live[pipe.tid] = "int64_t"
         cnt = pipe.reg("rcnt%d" % X, "uint32_t", "0", perRow=False)
@@ -225,7 +238,7 @@ class LaneRefill(UnaryTranslator):
         pipe.globalRefill = True
         pipe.phaseRows[1] = (cap, "std::min<uint64_t>(p.st->split_count[%d], p.gqcap%d)" % (idx, X))
         self._eagerAfterRelease(pipe)
-        self.parent.consume(ctxt)
+        self.above(ctxt)
 
     def _flushFlag(self, pipe, X, outer):
         if outer is None:
@@ -235,13 +248,17 @@ class LaneRefill(UnaryTranslator):
 
     def _consumeSmem(self, ctxt, pipe, X, live, cnt, thr, outer):
         nw = pipe.bs // 64
+        U = pipe.U
         queues = []
         for r, ct in live.items():
             q = "rq%d_%s" % (X, r)
-            pipe.staticLds.append("__shared__ %s %s[%d][128];" % (ct, q, nw))
+            # less than a threshold's worth waiting, and a trip's rows
+            pipe.staticLds.append("__shared__ %s %s[%d][%d];" % (ct, q, nw, 64 * (U + 1)))
             queues.append((r, q))
         pipe.emit("// lane refill (opId %d)" % X)
-        pipe.code.open("")
+        if U > 1:
+            pipe.emit("#pragma unroll")
+        pipe.code.open("for (int u = 0; u < %d; ++u)" % U if U > 1 else "")
         pipe.emit("const uint64_t rm = dqc::ballot(active[u]);")
         pipe.emit("const uint32_t rpos = %s + dqc::lanes_below(rm);" % cnt)
         pipe.code.open("if (active[u])")
@@ -249,15 +266,18 @@ class LaneRefill(UnaryTranslator):
             pipe.emit("%s[wave][rpos] = %s[u];" % (q, r))
         pipe.code.close()
         pipe.emit("%s += dqc::popc64(rm);" % cnt)
+        pipe.code.close()
         # entries written by some lanes are read back by others: order the
         # LDS stores before the pops below
         pipe.emit("dqc::wave_lds_sync();")
-        pipe.code.close()
         self._flushFlag(pipe, X, outer)
         point = {"id": X, "cnt": cnt}
         point["mark"] = pipe.code.mark()
         pipe.code.depth += 1
         pipe.refillPoints.append(point)
+        if U > 1:
+            pipe.U = 1
+            pipe.emit("constexpr int u = 0;")
         pipe.emit("const uint32_t rtake = %s < 64u ? %s : 64u;" % (cnt, cnt))
         pipe.emit("%s -= rtake;" % cnt)
         pipe.emit("active[u] = lane < rtake;")
@@ -269,9 +289,10 @@ class LaneRefill(UnaryTranslator):
         pipe.emit("dqc::wave_lds_sync();")
         point["cond"] = "%s >= (rflush%d ? 1u : %s)" % (cnt, X, thr)
         self._eagerAfterRelease(pipe)
-        self.parent.consume(ctxt)
+        self.above(ctxt)
         pipe.code.close()
-        pipe.emit("active[u] = 0;")
+        if U == 1:
+            pipe.emit("active[u] = 0;")
 
     def _consumeReg(self, ctxt, pipe, X, live, cnt, thr, outer):
         pipe.annotations.append("REG%d" % X)
@@ -316,7 +337,7 @@ class LaneRefill(UnaryTranslator):
         pipe.code.close()
         point["cond"] = go
         self._eagerAfterRelease(pipe)
-        self.parent.consume(ctxt)
+        self.above(ctxt)
         pipe.emit("active[u] = 0;")
         pipe.emit("%s = %s >= %s || (rflush%d && %s > 0u);" % (go, cnt, thr, X, cnt))
         pipe.code.close()

@@ -137,7 +137,8 @@ class Pipeline(object):
         self.bs = int(bs or KernelCall.defaultBlockSize)
         if self.bs % WAVE or not (WAVE <= self.bs <= 1024):
             raise ValueError("block size must be a multiple of 64 in [64, 1024]")
-        self.U = max(1, int(U))
+        self.U = max(1, int(U))     # rows per thread where code is being emitted (1 above a lane refill)
+        self.frontU = self.U        # rows per thread of a loop trip
         self.defaultGrid = int(KernelCall.defaultGridSize or 0)
         self.source = source
         self.params = OrderedDict()         # field -> (ctype, host expr)
@@ -274,7 +275,7 @@ class Pipeline(object):
 
     # ---- rendering
     def render(self):
-        U, B = self.U, self.bs
+        U, B = self.frontU, self.bs
         k = Code()
         k.open("struct KP_%s" % self.name)
         for f, (ct, _) in self.params.items():
@@ -595,6 +596,20 @@ class Program(object):
         h.emit("int64_t g = std::min<int64_t>(need, cap);")
         h.emit("return (unsigned)std::max<int64_t>(1, g);")
         h.close()
+        if any(p.refillPoints for p in self.pipes):
+            h.emit("// Workgroups of a pipeline with a lane refill: whole rounds of those that run at once,")
+            h.emit("// with rows enough for a wavefront to fill its queue more than it drains it")
+            h.open("static unsigned refillGrid(const void* kernel, int bs, size_t lds, int64_t rows)")
+            h.emit("int occ = 0;")
+            h.emit("if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kernel, bs, lds) != hipSuccess || occ < 1) "
+                   "{ (void)hipGetLastError(); occ = std::max(1, 1024 / bs); }")
+            h.emit("const int64_t resident = (int64_t)computeUnits() * occ, waves = bs / 64;")
+            h.emit("const int64_t many = rows / (waves * %d);" % REFILL_ROWS_MANY)
+            h.emit("if (many >= 2 * resident) return (unsigned)(many / resident * resident);")
+            h.emit("const int64_t few = std::min<int64_t>((rows + bs - 1) / bs, 4 * (int64_t)computeUnits());")
+            h.emit("return (unsigned)std::max<int64_t>(1, std::min<int64_t>(resident, "
+                   "std::max<int64_t>(few, rows / (waves * %d))));" % REFILL_ROWS)
+            h.close()
         h.open("static int computeLayout(const dqc_plan_inputs* in, const dqc_plan_tuning* t, Layout& L)")
         h.emit("if (!in || !t) return DQC_EINVAL;")
         h.emit("if (in->ntables != %d || in->ncols != %d) return DQC_EINVAL;" % (nt, nc))
@@ -806,10 +821,10 @@ def pipelineLaunch(prog, pipe, phase=None, rowsExpr=None, perCu=8):
         # the survivors' launch sizes its grid from the queue; the tuned grid
         # belongs to the first launch (with an LDS join filter, a few large
         # workgroups there)
-        lines.append("const unsigned g = gridFor(0, %s, %d, %s, %d, %d);" % (rows, pipe.bs, per, pipe.U, spread))
+        lines.append("const unsigned g = gridFor(0, %s, %d, %s, %d, %d);" % (rows, pipe.bs, per, pipe.frontU, spread))
     else:
         lines.append("const unsigned g = gridFor(t->grid[%d] > 0 ? t->grid[%d] : %d, %s, %d, %s, %d, %d);"
-                     % (pipe.pipeId, pipe.pipeId, pipe.defaultGrid, rows, pipe.bs, per, pipe.U, spread))
+                     % (pipe.pipeId, pipe.pipeId, pipe.defaultGrid, rows, pipe.bs, per, pipe.frontU, spread))
     if pipe.fewGroups:
         # rows enough for a workgroup to be worth its flush, every group of
         # its table: 8 per slot (a 246 k-row, 175-group group-by
@@ -834,6 +849,10 @@ def pipelineLaunch(prog, pipe, phase=None, rowsExpr=None, perCu=8):
         lines.append("kp.%s = 0u;" % pipe.ldsFilter["param"])
         lds = lds.replace(pipe.ldsFilter["host"], "(uint64_t)0")
     kname = pipe.name if phase is None else "%s<%d>" % (pipe.name, phase)
+    if pipe.refillPoints and phase is None and not pipe.defaultGrid:
+        lines = [ln.replace("const unsigned g", "unsigned g") for ln in lines]
+        lines.append("if (t->grid[%d] <= 0) g = refillGrid((const void*)&%s, %d, %s, %s);"
+                     % (pipe.pipeId, kname, pipe.bs, lds, rows))
     if pipe.dynLdsExpr is not None:
         # dynamic LDS beyond 64 KB (gfx950 has 160 KB per workgroup) is opted into per kernel
         lines.append("if (%s > 65536u) (void)hipFuncSetAttribute((const void*)&%s, "
@@ -1077,8 +1096,45 @@ def lineTouchFraction(rowFraction, elemBytes, lineBytes=128):
 
 
 def rowsPerThread(translator):
-    loops, _ = pipelineShape(translator)
-    return 1 if loops else max(1, int(KernelCall.defaultRowsPerThread))
+    U = max(1, int(KernelCall.defaultRowsPerThread))
+    if not pipelineShape(translator)[0]:
+        return U
+    # Up to a lane refill in LDS a pipeline can carry rows side by side (their
+    # loads are in flight together, and the queue takes them one after
+    # another); above it, and with any other loop, it is one row per lane.
+    # FIGURES
+    return min(U, FRONT_ROWS) if _refillFirst(translator) else 1
+
+
+FRONT_ROWS = 4
+# rows per wavefront of a pipeline with a lane refill: in one round of
+# workgroups at least the first, in several about the second.  A round that is
+# partly empty costs as much as a full one, and a wavefront with few rows mostly
+# drains: c3's sales kernel at 60 M rows, 5 workgroups per CU at once, 2048
+# workgroups 623 us, 1024 560, 8960 (7 rounds) 465; at 4.6 M rows 2048 48 us,
+# 8192 115, 1280 42; TPC-H Q10's lineitem kernel 2048 219 us, one round 192.
+REFILL_ROWS, REFILL_ROWS_MANY = 512, 1536
+
+
+def _refillFirst(translator):
+    """The first operator of the pipeline that loops per lane is a lane
+    refill with the LDS queue."""
+    from dogqc_amd.hashJoins import EquiJoinTranslator
+    from dogqc_amd.hipDivergenceBuffer import LaneRefill, BufferType
+    from dogqc_amd.relationalAlgebra import Join
+    t = translator
+    while t.parent is not None:
+        p = t.parent
+        if isinstance(p, LaneRefill):
+            return p.bufferType is BufferType.SMEM
+        if isinstance(p, BinaryTranslator) and p.leftChild is t:
+            return False
+        if isinstance(p, CrossJoinTranslator):
+            return False
+        if isinstance(p, EquiJoinTranslator) and p.algExpr.multimatch and p.algExpr.joinType in (Join.INNER, Join.OUTER):
+            return False
+        t = p
+    return False
 
 
 def launchShape(translator):

@@ -85,3 +85,28 @@ def test_ranked_rows(orders, grid):
         t.grid[i] = grid
     for q in ("tpch13", "tpch16"):
         check(q, acc, tuning=t, label="orders=%d" % orders)
+
+
+# lane refill behind several rows per thread, with the refill above a filtered
+# join placed between the filter and the probe: trips' edges, thresholds, and
+# the filter off, in LDS and in device memory
+@pytest.mark.gpu
+@pytest.mark.parametrize("plan", ["c1_refill", "c3_refill", "tpch10", "f_like_project_refill"])
+@pytest.mark.parametrize("n", [1, 257, 3071, 3073, 9000])
+def test_refill_front(plan, n):
+    from dogqc_amd import tpch
+    from dogqc_amd.dbio import MemoryAccessor
+    if plan == "tpch10":
+        acc = MemoryAccessor(tpch.generate(n / 6.0e6, seed=n))
+    elif plan == "c1_refill":
+        acc = workloadAcc("c1", {"dim": max(1, n // 4), "fact": n}, seed=n)
+    elif plan == "c3_refill":
+        acc = workloadAcc("c3", {"sales": n, "item": max(1, n // 20), "cust": max(1, n // 50)}, seed=n)
+    else:
+        acc = planlib.featureData(n, 10, seed=n)
+    for grid, threshold, jf in ((0, 0, 0), (GRID, 1, 0), (GRID, 64, -1), (GRID, 0, 32), (1, 0, 1024), (5000, 64, 0)):
+        t = rt.newTuning()
+        t.join_filter = jf
+        for i in range(rt.MAX_PIPES):
+            t.grid[i], t.refill_threshold[i] = grid, threshold
+        check(plan, acc, tuning=t, label="n=%d grid=%d threshold=%d filter=%d" % (n, grid, threshold, jf))
