@@ -237,7 +237,7 @@ class EquiJoinTranslator(BinaryTranslator):
                 "L.mment[%d] = t->mm_entries[%d] > 0 ? t->mm_entries[%d] : std::max<int64_t>(64, %s * 2);\n"
                 "if (L.mment[%d] >= (int64_t)0xffffffffll) return DQC_ENOMEM;" % (idx, idx, idx, est, idx))
             dirb = prog.buffer("jht%d_dir" % J, CType.UINT, "2 * L.htcap[%d]" % idx, "0x0ull")
-            sums = prog.buffer("jht%d_sums" % J, CType.UINT64, "(L.htcap[%d] + 4095) / 4096 + 1" % idx)
+            sums = prog.buffer("jht%d_sums" % J, CType.UINT64, "(L.htcap[%d] + 4095) / 4096 + 2" % idx, "0x0ull")
             ht["dirBuffer"], ht["sumsBuffer"] = dirb, sums
             fdir = pipe.param("jht%d_dir" % J, "uint32_t*", "B_" + dirb)
             fcap = pipe.param("jht%d_cap" % J, "uint32_t", "L.htcap[%d]" % idx)

@@ -1330,29 +1330,16 @@ def closePipeline(ctxt, pipe):
 
 
 def mmScanSteps(ht):
-    """Bucket-count exclusive scan of a multimap (three kernels)."""
+    """Bucket-count exclusive scan of a multimap."""
     dirb, sums, idx = ht["dirBuffer"], ht["sumsBuffer"], ht["index"]
 
-    def reduce_(prog):
+    def scan(prog):
         return ["const uint64_t nb = (uint64_t)L.htcap[%d];" % idx,
                 "const unsigned g = (unsigned)std::max<uint64_t>(1, (nb + dqc::SCAN_TILE - 1) / dqc::SCAN_TILE);",
-                "hipLaunchKernelGGL(dqc::dqc_mm_scan_reduce, dim3(g), dim3(dqc::SCAN_BS), 0, s, "
-                "(const uint32_t*)B_%s, nb, B_%s);" % (dirb, sums)]
+                "hipLaunchKernelGGL(dqc::dqc_mm_scan, dim3(g), dim3(dqc::SCAN_BS), 0, s, (uint32_t*)B_%s, nb, B_%s, g, "
+                "&st->mm_total[%d], %du);" % (dirb, sums, idx, 1 if ht.get("ranked") else 0)]
 
-    def blocks(prog):
-        return ["const uint64_t nb = (uint64_t)L.htcap[%d];" % idx,
-                "const uint64_t g = std::max<uint64_t>(1, (nb + dqc::SCAN_TILE - 1) / dqc::SCAN_TILE);",
-                "hipLaunchKernelGGL(dqc::dqc_mm_scan_blocks, dim3(1), dim3(dqc::SCAN_BS), 0, s, B_%s, g, "
-                "&st->mm_total[%d]);" % (sums, idx)]
-
-    def apply_(prog):
-        return ["const uint64_t nb = (uint64_t)L.htcap[%d];" % idx,
-                "const unsigned g = (unsigned)std::max<uint64_t>(1, (nb + dqc::SCAN_TILE - 1) / dqc::SCAN_TILE);",
-                "hipLaunchKernelGGL(dqc::dqc_mm_scan_apply, dim3(g), dim3(dqc::SCAN_BS), 0, s, "
-                "(uint32_t*)B_%s, nb, (const uint64_t*)B_%s, %du);" % (dirb, sums, 1 if ht.get("ranked") else 0)]
-
-    return [{"name": "dqc_mm_scan_reduce", "host": reduce_}, {"name": "dqc_mm_scan_blocks", "host": blocks},
-            {"name": "dqc_mm_scan_apply", "host": apply_}]
+    return [{"name": "dqc_mm_scan", "host": scan}]
 
 
 class SelectionTranslator(UnaryTranslator):
