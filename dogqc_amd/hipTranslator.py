@@ -159,6 +159,8 @@ class Pipeline(object):
         self.refillPoints = []
         self.annotations = []
         self.fewGroups = False       # ends in a group-by known to have few groups (launchShape)
+        self.gatherAt = None         # push-down probe that gathers its rows (EquiJoinTranslator.gathers)
+        self.drains = False          # its queue is emptied in one more trip after the last rows
         self.rankedRows = False      # the second launch reads which rows passed the filters
         self.sharedAtomics = False   # every workgroup updates the same few words
         self.innerDepth = 0
@@ -333,21 +335,25 @@ class Pipeline(object):
         if pa is not None:
             first, step, trip = ["PHASE == 1 ? %s : %s" % (x, y) for x, y in
                                  (("0", first), ("(int64_t)%d" % B, step), ("(int64_t)%d" % (B * U), trip))]
+        elif self.drains and U > 1:
+            # (the second launch takes one chunk of a list per thread and trip)
+            first, trip = ["PHASE == 1 ? %s : %s" % (x, y) for x, y in
+                           (("(int64_t)blockIdx.x * %d" % B, first), ("(int64_t)gridDim.x * %d" % B, trip))]
         k.emit("const int64_t step = %s, trip = %s;" % (step, trip))
         # (lane refills drain their buffers in one more trip, after the last rows)
-        k.open("for (int64_t base = %s;%s; base += trip)" % (first, "" if self.refillPoints else " base < nrows"))
+        k.open("for (int64_t base = %s;%s; base += trip)" % (first, "" if self.refillPoints or self.drains else " base < nrows"))
         k.emit("const bool more = base < nrows;")
         k.emit("int active[%d];" % U)
         if U > 1:
             k.emit("#pragma unroll")
             k.open("for (int u = 0; u < %d; ++u)" % U)
         k.emit("%s[u] = base%s + (int64_t)threadIdx.x;" % (self.tid, " + u * step" if U > 1 else ""))
-        k.emit("active[u] = more && %s[u] < nrows;" % self.tid)
+        k.emit("active[u] = more && %s[u] < nrows%s;" % (self.tid, " && (PHASE == 0 || u == 0)" if self.drains and U > 1 else ""))
         if U > 1:
             k.close()
         k.extend(self.code)
         k.extend(self.iterationEnd)
-        if self.refillPoints:
+        if self.refillPoints or self.drains:
             k.emit("if (!more) break;")
         k.close()
         k.extend(self.epilogue)
@@ -596,7 +602,7 @@ class Program(object):
         h.emit("int64_t g = std::min<int64_t>(need, cap);")
         h.emit("return (unsigned)std::max<int64_t>(1, g);")
         h.close()
-        if any(p.refillPoints for p in self.pipes):
+        if any(p.refillPoints or p.drains for p in self.pipes):
             h.emit("// Workgroups of a pipeline with a lane refill: whole rounds of those that run at once,")
             h.emit("// with rows enough for a wavefront to fill its queue more than it drains it")
             h.open("static unsigned refillGrid(const void* kernel, int bs, size_t lds, int64_t rows)")
@@ -823,8 +829,9 @@ def pipelineLaunch(prog, pipe, phase=None, rowsExpr=None, perCu=8):
         # workgroups there)
         lines.append("const unsigned g = gridFor(0, %s, %d, %s, %d, %d);" % (rows, pipe.bs, per, pipe.frontU, spread))
     else:
+        U = 1 if pipe.drains and phase == 1 else pipe.frontU
         lines.append("const unsigned g = gridFor(t->grid[%d] > 0 ? t->grid[%d] : %d, %s, %d, %s, %d, %d);"
-                     % (pipe.pipeId, pipe.pipeId, pipe.defaultGrid, rows, pipe.bs, per, pipe.frontU, spread))
+                     % (pipe.pipeId, pipe.pipeId, pipe.defaultGrid, rows, pipe.bs, per, U, spread))
     if pipe.fewGroups:
         # rows enough for a workgroup to be worth its flush, every group of
         # its table: 8 per slot (a 246 k-row, 175-group group-by
@@ -849,7 +856,7 @@ def pipelineLaunch(prog, pipe, phase=None, rowsExpr=None, perCu=8):
         lines.append("kp.%s = 0u;" % pipe.ldsFilter["param"])
         lds = lds.replace(pipe.ldsFilter["host"], "(uint64_t)0")
     kname = pipe.name if phase is None else "%s<%d>" % (pipe.name, phase)
-    if pipe.refillPoints and phase is None and not pipe.defaultGrid:
+    if ((pipe.refillPoints and phase is None) or (pipe.drains and phase == 0)) and not pipe.defaultGrid:
         lines = [ln.replace("const unsigned g", "unsigned g") for ln in lines]
         lines.append("if (t->grid[%d] <= 0) g = refillGrid((const void*)&%s, %d, %s, %s);"
                      % (pipe.pipeId, kname, pipe.bs, lds, rows))
@@ -1103,7 +1110,7 @@ def rowsPerThread(translator):
     # loads are in flight together, and the queue takes them one after
     # another); above it, and with any other loop, it is one row per lane.
     # FIGURES
-    return min(U, FRONT_ROWS) if _refillFirst(translator) else 1
+    return min(U, FRONT_ROWS) if _refillFirst(translator) or gatheringProbe(translator) is not None else 1
 
 
 FRONT_ROWS = 4
@@ -1114,6 +1121,28 @@ FRONT_ROWS = 4
 # workgroups 623 us, 1024 560, 8960 (7 rounds) 465; at 4.6 M rows 2048 48 us,
 # 8192 115, 1280 42; TPC-H Q10's lineitem kernel 2048 219 us, one round 192.
 REFILL_ROWS, REFILL_ROWS_MANY = 512, 1536
+
+
+def gatheringProbe(translator):
+    """The pipeline's first operator that moves rows between lanes, if it is
+    a push-down probe that gathers its rows; else None."""
+    from dogqc_amd.hashJoins import EquiJoinTranslator
+    from dogqc_amd.hipDivergenceBuffer import LaneRefill
+    from dogqc_amd.relationalAlgebra import Join
+    t, fraction = translator, 1.0
+    while t.parent is not None:
+        p = t.parent
+        if isinstance(p, (LaneRefill, CrossJoinTranslator)) or (isinstance(p, BinaryTranslator) and p.leftChild is t):
+            return None
+        if isinstance(p, SelectionTranslator):
+            fraction *= float(getattr(p.algExpr, "selectivity", 1.0))
+        elif isinstance(p, EquiJoinTranslator):
+            if p.algExpr.multimatch and p.algExpr.joinType in (Join.INNER, Join.OUTER):
+                return p if p.gathers(fraction) else None
+            if p.algExpr.joinType in (Join.INNER, Join.SEMI):
+                fraction *= min(1.0, float(getattr(p.algExpr, "selectivity", 1.0)))
+        t = p
+    return None
 
 
 def _refillFirst(translator):
@@ -1267,6 +1296,7 @@ class ScanTranslator(LiteralTranslator):
             with pipe.rowLoop():
                 pipe.emit("if (active[u]) active[u] = %s[%s[u]] != 0xffffffffu;" % (f, pipe.tid))
             pipe.code.close()
+        pipe.gatherAt = gatheringProbe(self)
         fracs = firstUseFractions(self)
         eager = []
         for id, attr in self.algExpr.outRelation.items():
