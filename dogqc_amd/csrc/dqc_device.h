@@ -248,11 +248,6 @@ DQC_DEVICE_INLINE int64_t ht_insert_from(Tag* tags, uint32_t cap, Tag tag, uint3
     return -1;
 }
 
-DQC_DEVICE_INLINE int64_t ht_insert(uint64_t* tags, uint32_t cap, uint64_t tag, uint64_t h,
-                                    const uint32_t* status) {
-    return ht_insert_from<uint64_t>(tags, cap, tag, slot_of(h, cap), 0u, status);
-}
-
 // A join probe starts here.
 DQC_DEVICE_INLINE uint32_t probe_start(uint64_t h, uint32_t cap) { return slot_of(h, cap); }
 

@@ -291,6 +291,7 @@ class EquiJoinTranslator(BinaryTranslator):
             if self._buildPartitionable(pipe):
                 self._partitionedBuild(ctxt, pipe, prog, ins, est)
             else:
+                pipe.scatters = self._scansIntoBuild()
                 self._directInsert(pipe, ins, "active[u]")
             return
         # multimap: count pass (PHASE 0) and insert pass (PHASE 1) of one kernel
@@ -327,6 +328,15 @@ class EquiJoinTranslator(BinaryTranslator):
 
     def _packedWord(self, pipe, jtag):
         return "dqc::packed_slot(%s, dqc::to_word<%s>(%s))" % (jtag, self.packedType, pipe.access(self.stored[0]))
+
+    def _scansIntoBuild(self):
+        """Nothing but filters and expressions between a table's scan and this
+        build: rows are inserted straight from it."""
+        from dogqc_amd.hipTranslator import MapTranslator, ScanTranslator, SelectionTranslator
+        t = self.leftChild
+        while isinstance(t, (SelectionTranslator, MapTranslator)):
+            t = t.child
+        return isinstance(t, ScanTranslator)
 
     def _firstCas(self, pipe, ins):
         """Home slot and first CAS of a row whose tag and hash jhJ are set."""

@@ -163,6 +163,7 @@ class Pipeline(object):
         self.drains = False          # its queue is emptied in one more trip after the last rows
         self.rankedRows = False      # the second launch reads which rows passed the filters
         self.sharedAtomics = False   # every workgroup updates the same few words
+        self.scatters = False        # ends in inserts all over a join table
         self.innerDepth = 0
         self.probedJoins = []
         self.loopInvariant = None   # attribute ids loaded before the per-lane match loop being emitted
@@ -814,6 +815,15 @@ def pipelineLaunch(prog, pipe, phase=None, rowsExpr=None, perCu=8):
     # there took c1's 600 k-slot output kernel (an append) from 14.4 to 30.2 us
     # and c2's count pass (1 M rows) from 52.8 to 74.5 us.
     spread = 1 if pipe.sharedAtomics else perCu
+    # One that inserts a table's rows into a join table waits for a row's first
+    # CAS before the next row's and has nothing that a workgroup pays once: four
+    # times as many, down to a row per thread.  c1's build (4.2 M rows scanned)
+    # 38.7 -> 31.5 us, c3's item build at 15 M rows 58.3 -> 50.8; 80 k rows the
+    # same.  With a probe before the insert few rows are left to wait for: Q18's
+    # orders kernel 30.4 -> 33.5 us.
+    if pipe.scatters and not pipe.sharedAtomics:
+        spread = 4 * perCu
+        per = str(spread)
     lds = "0" if pipe.dynLdsExpr is None else "(size_t)(%s)" % pipe.dynLdsExpr
     pa = pipe.partAgg
     if pa is not None and phase == 0:
@@ -1109,7 +1119,7 @@ def rowsPerThread(translator):
     # Up to a lane refill in LDS a pipeline can carry rows side by side (their
     # loads are in flight together, and the queue takes them one after
     # another); above it, and with any other loop, it is one row per lane.
-    # FIGURES
+    # (Q10's lineitem kernel 247 -> 221 us with four, c2's count pass 124 -> 97.)
     return min(U, FRONT_ROWS) if _refillFirst(translator) or gatheringProbe(translator) is not None else 1
 
 

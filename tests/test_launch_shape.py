@@ -110,3 +110,18 @@ def test_refill_front(plan, n):
         for i in range(rt.MAX_PIPES):
             t.grid[i], t.refill_threshold[i] = grid, threshold
         check(plan, acc, tuning=t, label="n=%d grid=%d threshold=%d filter=%d" % (n, grid, threshold, jf))
+
+
+def test_join_builds_take_a_row_per_thread():
+    """A pipeline that ends in inserts into a join table is launched on four
+    times the workgroups of the others."""
+    src = planlib.translate("c1").source
+    host = [ln for ln in src.splitlines() if "gridFor(t->grid[" in ln]
+    assert host[0].split("gridFor")[1].endswith(", 256, 32, 4, 32);") and not any("32, 4, 32" in ln for ln in host[1:])
+
+
+# the build's grid ends at 256 CUs x 32 workgroups x 256 rows
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [2048 * 256 + 1, 8192 * 256 - 1, 8192 * 256 + 1, 8192 * 1024 + 257])
+def test_join_build_grid(n):
+    check("c1", workloadAcc("c1", {"dim": n, "fact": 1 << 16}, seed=n % 97), label="dim=%d" % n)
