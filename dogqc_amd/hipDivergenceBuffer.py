@@ -11,9 +11,10 @@ Two buffer kinds, selected like the reference's BufferType
 (cudaDivergenceBuffer.py:44-46) through ``LaneRefill.bufferType``:
 
 * ``BufferType.SMEM`` (default): every wavefront owns an LDS queue per live
-  register (64 entries and 64 more per row that a thread carries up to here) (attributes already in registers, plus the row indices
-  of attributes that are still loaded lazily, so columns that only later
-  operators read are fetched after compaction, for dense lanes only).
+  register, of 64 entries and 64 more per row that a thread carries up to
+  here.  Live registers are the attributes already in registers, plus the row
+  indices of attributes that are still loaded lazily, so columns that only
+  later operators read are fetched after compaction, for dense lanes only.
   Survivors are appended with one 64-bit ballot and an mbcnt prefix; the
   downstream code runs on up to 64 popped entries at a time.
 

@@ -1120,9 +1120,42 @@ def rowsPerThread(translator):
     # loads are in flight together, and the queue takes them one after
     # another); above it, and with any other loop, it is one row per lane.
     # (Q10's lineitem kernel 247 -> 221 us with four, c2's count pass 124 -> 97.)
-    return min(U, FRONT_ROWS) if _refillFirst(translator) or gatheringProbe(translator) is not None else 1
+    # A row of the queue holds at most queuedBytes, and a wavefront
+    # 64 rows and 64 more per row that a thread carries.
+    if not (_refillFirst(translator) or gatheringProbe(translator) is not None):
+        return 1
+    rowBytes = (int(KernelCall.defaultBlockSize) // WAVE) * WAVE * queuedBytes(translator)
+    return max(1, min(U, FRONT_ROWS, QUEUE_LDS // rowBytes - 1))
 
 
+def queuedBytes(translator):
+    """At most the bytes of a row's registers that a queue at the pipeline's
+    first lane refill or gathering probe holds: the attributes that reach it
+    and the row and slot indices of those not loaded yet."""
+    from dogqc_amd.hashJoins import EquiJoinTranslator
+    from dogqc_amd.hipDivergenceBuffer import LaneRefill
+    size = lambda a: 16 if a.dataType == Type.STRING else COLUMN_BYTES.get(a.dataType, 8)
+    attrs, t, indices = {}, translator, 8
+    while t is not None and not isinstance(t, LaneRefill):
+        out = t.algExpr.outRelation
+        if isinstance(t, EquiJoinTranslator):
+            # (tag, slot, null flag, the column of a packed slot)
+            indices += 8 + 8 + 4 + 4
+            if isinstance(t.parent, LaneRefill):
+                # nothing has read the build side's columns yet
+                out = {i: a for i, a in out.items() if i not in t.algExpr.leftChild.outRelation}
+            else:
+                attrs.update(t.algExpr.leftChild.outRelation)
+        attrs.update(out)
+        if isinstance(t, EquiJoinTranslator) and t.algExpr.multimatch:
+            break
+        t = t.parent
+    return indices + sum(size(a) for a in attrs.values())
+
+
+# LDS that the queues of a workgroup with several rows per thread may take: two
+# such workgroups fit a CU (160 KB)
+QUEUE_LDS = 80 << 10
 FRONT_ROWS = 4
 # rows per wavefront of a pipeline with a lane refill: in one round of
 # workgroups at least the first, in several about the second.  A round that is
@@ -2165,7 +2198,8 @@ class AggregationTranslator(UnaryTranslator):
         pipe.code.lines.insert(0, "    " * (pipe.code.depth - 1) + "if constexpr (PHASE == 0) {")
         pipe.code.depth += 1
         pipe.code.open("if (%s == 0u)" % fnp)
-        self._exactUpdate(pipe, tagCode, vals, upd, "gh")
+        # (without partitions the table is one range)
+        self._exactUpdate(pipe, tagCode, vals, dict(upd, range=None), "gh")
         pipe.code.close()
         pipe.code.open("else")
         pipe.emit("// append to this workgroup's segment of the row's partition")

@@ -112,6 +112,25 @@ def test_refill_front(plan, n):
         check(plan, acc, tuning=t, label="n=%d grid=%d threshold=%d filter=%d" % (n, grid, threshold, jf))
 
 
+@pytest.mark.parametrize("plan", ["c2_pushdown", "c2_both", "c3_refill", "f_like_project_refill", "tpch3", "tpch5",
+                                  "tpch7", "tpch8", "tpch9", "tpch10", "tpch14", "tpch19"])
+@pytest.mark.parametrize("budget", [80 << 10, 40 << 10, 16 << 10, 0])
+def test_queue_stays_in_its_lds(plan, budget, monkeypatch):
+    """A queue holds no more per row than the bound that chose the rows per
+    thread, so it keeps to its share of LDS (or to one row per thread)."""
+    from dogqc_amd import hipTranslator as H
+    monkeypatch.setattr(H, "QUEUE_LDS", budget)
+    bounds, bound = [], H.queuedBytes
+    monkeypatch.setattr(H, "queuedBytes", lambda t: bounds.append(bound(t)) or bounds[-1])
+    for pipe in planlib.translate(plan).program.pipes:
+        if not (pipe.refillPoints or pipe.drains):
+            continue
+        pipe.staticLds = [d for d in pipe.staticLds if d.split()[2].startswith(("rq", "pg"))]
+        rows = (pipe.bs // 64) * 64 * (pipe.frontU + 1)
+        assert H.staticLdsBytes(pipe) <= rows * sum(bounds), (plan, bounds)
+        assert pipe.frontU == 1 or rows * max(bounds) <= budget
+
+
 def test_join_builds_take_a_row_per_thread():
     """A pipeline that ends in inserts into a join table is launched on four
     times the workgroups of the others."""
