@@ -73,7 +73,7 @@ typedef struct dqc_plan_inputs {
  * cfg htSizeFactor (relationalAlgebra.py:453-455) with per-pipeline values. */
 typedef struct dqc_plan_tuning {
     int32_t grid[DQC_MAX_PIPES];             /* workgroups per pipeline kernel */
-    int32_t refill_threshold[DQC_MAX_PIPES]; /* 1..64 active lanes */
+    int32_t refill_threshold[DQC_MAX_PIPES]; /* 1..64 active lanes (lane refills, push-down probes that gather) */
     int32_t lds_slots[DQC_MAX_PIPES];        /* LDS group slots (power of 2); -1 = no LDS tier */
     int32_t lds_replicas[DQC_MAX_PIPES];     /* LDS accumulator replicas (power of 2, <= 64) */
     float ht_factor[DQC_MAX_HTS];            /* multiplies htSizeFactor / the 2x agg factor */
@@ -90,9 +90,12 @@ typedef struct dqc_plan_tuning {
                                                 into dqc_plan_status.ht_fill after the plan */
     int32_t part_agg;                        /* partitioned group-by (plans translated with it): 0 = when
                                                 the group count (ht_capacity / 2, else the plan's numgroups)
-                                                exceeds 16384, -1 = never, n > 0 = n partitions */
-    int32_t join_filter;                     /* LDS filter of the build keys of selective unique joins
-                                                (plans translated with it): n > 0 = n KB, else none */
+                                                exceeds 2048 and the input 65536 rows, -1 = never,
+                                                n > 0 = n partitions */
+    int32_t join_filter;                     /* filter of the build keys of selective unique joins: n > 0 =
+                                                n KB (in LDS when it fits), 0 = 16 bits per key in device
+                                                memory for a join whose lane refill gathers the rows that
+                                                pass it, else the plan's default; < 0 = none */
     int32_t part_build;                      /* partitioned unique-join build (plans translated with it):
                                                 n > 0 = n partitions, else none */
     int32_t reserved[2];
@@ -194,7 +197,8 @@ typedef struct dqc_query_result {
     int32_t retries;
 } dqc_query_result;
 
-/* Run a plan to completion on `stream`: allocate the workspace, enqueue,
+/* Run a plan to completion on `stream`: allocate the workspace (a released
+ * one of about the size if there is one, dqc_query_release), enqueue,
  * synchronise, and on a full hash table, multimap, temp table or result buffer enlarge
  * it (tuning is updated in place) and run again, up to max_retries times. */
 int dqc_query_run(void* module, const dqc_plan_inputs* in, dqc_plan_tuning* tun, void* stream,
