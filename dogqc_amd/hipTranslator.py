@@ -286,7 +286,14 @@ class Pipeline(object):
         k.close(";")
         if self.phased:
             k.emit("template <int PHASE>")
-        k.open("__global__ void __launch_bounds__(%d) %s(const KP_%s p)" % (B, self.name, self.name))
+        # A SIMD holds 8 waves of up to 80 scalar registers (96 with what the trap
+        # handler reserves, of 800) and 7 of up to 96: with large workgroups that
+        # is one workgroup in two.  Q15's lineitem kernel at 1024 threads, 42
+        # vector and 87 scalar registers, 40.5 us without the limit, 29.2 with
+        # it; c3's by-item aggregation 64.5 -> 52.9.  Not where one workgroup
+        # per CU runs anyway: there it only spills (TPC-H Q1 269 -> 276 us).
+        sgprs = " __attribute__((amdgpu_num_sgpr(80)))" if B >= 512 and not self.fewGroups else ""
+        k.open("__global__ void __launch_bounds__(%d)%s %s(const KP_%s p)" % (B, sgprs, self.name, self.name))
         for d in self.staticLds:
             k.emit(d)
         if self.dynLdsExpr is not None:

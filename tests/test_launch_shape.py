@@ -144,3 +144,11 @@ def test_join_builds_take_a_row_per_thread():
 @pytest.mark.parametrize("n", [2048 * 256 + 1, 8192 * 256 - 1, 8192 * 256 + 1, 8192 * 1024 + 257])
 def test_join_build_grid(n):
     check("c1", workloadAcc("c1", {"dim": n, "fact": 1 << 16}, seed=n % 97), label="dim=%d" % n)
+
+
+def test_scalar_registers_of_large_workgroups():
+    """Large workgroups that share a CU are limited to 80 scalar registers."""
+    few, many, small = planlib.translate("tpch1").source, planlib.translate("tpch18").source, planlib.translate("c1").source
+    assert "__launch_bounds__(1024) krnl_lineitem1(" in few
+    assert "__launch_bounds__(1024) __attribute__((amdgpu_num_sgpr(80))) krnl_lineitem1(" in many
+    assert "amdgpu_num_sgpr" not in small
