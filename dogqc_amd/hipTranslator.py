@@ -1182,7 +1182,8 @@ def gatheringProbe(translator):
     t, fraction = translator, 1.0
     while t.parent is not None:
         p = t.parent
-        if isinstance(p, (LaneRefill, CrossJoinTranslator)) or (isinstance(p, BinaryTranslator) and p.leftChild is t):
+        if isinstance(p, (LaneRefill, CrossJoinTranslator, AggregationTranslator, MaterializeTranslator)) or \
+                (isinstance(p, BinaryTranslator) and p.leftChild is t):
             return None
         if isinstance(p, SelectionTranslator):
             fraction *= float(getattr(p.algExpr, "selectivity", 1.0))
@@ -1268,6 +1269,15 @@ def _groupsAbove(translator):
     return None
 
 
+def openPipeline(prog, translator, name, source):
+    """A pipeline that `translator` (a scan of a table, a temp table or a
+    group table) feeds.  Its launch shape counts on a probe that gathers, so
+    the two are set together."""
+    pipe = prog.newPipeline(name, source, *launchShape(translator))
+    pipe.gatherAt = gatheringProbe(translator)
+    return pipe
+
+
 class ScanTranslator(LiteralTranslator):
     """Opens a pipeline over a base table.  Columns load lazily at first use,
     except those whose cache lines would nearly all be read anyway: a column
@@ -1291,8 +1301,7 @@ class ScanTranslator(LiteralTranslator):
             self._produceTemp(ctxt, name)
             return
         ti = prog.table(tname)
-        pipe = prog.newPipeline(name, {"rows": "L.rows[%d]" % ti, "tidName": "%s%d" % (tname, a.scanTableId)},
-                                *launchShape(self))
+        pipe = openPipeline(prog, self, name, {"rows": "L.rows[%d]" % ti, "tidName": "%s%d" % (tname, a.scanTableId)})
         pipe.scanTable = tname
         ctxt.pipe = pipe
         tid = pipe.tid + "[u]"
@@ -1346,7 +1355,6 @@ class ScanTranslator(LiteralTranslator):
             with pipe.rowLoop():
                 pipe.emit("if (active[u]) active[u] = %s[%s[u]] != 0xffffffffu;" % (f, pipe.tid))
             pipe.code.close()
-        pipe.gatherAt = gatheringProbe(self)
         fracs = firstUseFractions(self)
         eager = []
         for id, attr in self.algExpr.outRelation.items():
@@ -1372,8 +1380,8 @@ class ScanTranslator(LiteralTranslator):
         if tmp is None:
             raise ValueError("temp table %s is scanned before it is created" % a.table["name"])
         ti = tmp["index"]
-        pipe = prog.newPipeline(name, {"rows": "L.tcap[%d]" % ti, "devRows": "st->temp_count[%d]" % ti,
-                                       "tidName": "%s%d" % (a.table["name"], a.scanTableId)}, *launchShape(self))
+        pipe = openPipeline(prog, self, name, {"rows": "L.tcap[%d]" % ti, "devRows": "st->temp_count[%d]" % ti,
+                                               "tidName": "%s%d" % (a.table["name"], a.scanTableId)})
         ctxt.pipe = pipe
         tid = pipe.tid + "[u]"
         byName = {c["name"]: c for c in tmp["columns"]}
@@ -2451,7 +2459,7 @@ class AggregationTranslator(UnaryTranslator):
         rows = "L.htcap[%d]" % (self.fused["htIndex"] if self.fused else self.ht["index"])
         if (self.fused is None and self.doGroup and self.exact64) or (self.fused is not None and self.fused["tag32"]):
             rows += " + 1"     # the extra slot
-        pipe = prog.newPipeline(name, {"rows": rows, "tidName": "agg%d" % a.opId}, *launchShape(self))
+        pipe = openPipeline(prog, self, name, {"rows": rows, "tidName": "agg%d" % a.opId})
         ctxt.pipe = pipe
         tid = pipe.tid + "[u]"
         pipe.param("st", "dqc_plan_status*", "st")

@@ -170,6 +170,17 @@ def _featurePlan(name, alg):
                            alg.join(("u_grp", "t_grp"), alg.scan("u"),
                                     alg.selection(scal.SmallerExpr(_A("t_id"), _C("300", Type.INT)), alg.scan("t"))))
         return p, {4: {"multimatch": True}}
+    if name in ("f_group_probe", "f_group_refill"):
+        # a group table as the source of a probe that few of its rows reach:
+        # of a multimap (a push-down probe gathers the rows first) or, with
+        # the lane refill at the selection, of a unique table
+        p = alg.projection(["t_grp", "c", "mv", "u_id", "u_w"],
+                           alg.join(("u_grp" if name == "f_group_probe" else "u_id", "t_grp"), alg.scan("u"),
+                                    alg.selection(scal.LargerExpr(_A("c"), _C("42", Type.INT)),
+                                                  alg.aggregation(["t_grp"], [(Reduction.COUNT, "", "c"),
+                                                                              (Reduction.MAX, "t_val", "mv")],
+                                                                  alg.scan("t")))))
+        return p, {4: {"selectivity": 0.1}, 5: {"multimatch": name == "f_group_probe"}}
     if name == "f_join_string":
         # multimatch join on a string key (single-word t_txt = u_name, about
         # 70 u rows per word), grouped by t_cat
@@ -390,7 +401,7 @@ FEATURE_PLANS = ["f_scan_minmax", "f_groupby_hashed", "f_groupby_wide", "f_like_
                  "f_join_unique_lowest",
                  "f_groupjoin", "f_join_multi", "f_semi", "f_anti_multi", "f_temp", "f_temp_strings", "f_groupby_64",
                  "f_groupby_int64", "f_outer", "f_outer_project", "f_join_neg", "f_anti_neg",
-                 "f_join_packed", "f_cross", "f_cross_pairs", "f_like_patterns", "f_join_string"]
+                 "f_join_packed", "f_cross", "f_cross_pairs", "f_like_patterns", "f_join_string", "f_group_probe"]
 
 # name -> (workload or "feature", options)
 PLANS = OrderedDict()
@@ -417,6 +428,8 @@ for _n in FEATURE_PLANS:
 for _n in STRING_PLANS:
     PLANS[_n] = ("strings", {})
 PLANS["f_join_multi_pushdown"] = ("feature", {"pushdown": True, "base": "f_join_multi"})
+PLANS["f_group_probe_pushdown"] = ("feature", {"pushdown": True, "base": "f_group_probe"})
+PLANS["f_group_refill"] = ("feature", {"buffers": [4]})
 PLANS["f_join_string_pushdown"] = ("feature", {"pushdown": True, "base": "f_join_string"})
 # string keys hashed and compared by the whole wavefront (StringHash.wave)
 PLANS["f_join_string_ws"] = ("feature", {"wave_strings": True, "base": "f_join_string"})
