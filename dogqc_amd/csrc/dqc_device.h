@@ -24,6 +24,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <cmath>
+
 #ifndef DQC_DEVICE_INLINE
 #define DQC_DEVICE_INLINE __device__ __forceinline__
 #endif
@@ -446,6 +448,16 @@ DQC_DEVICE_INLINE uint32_t part_home(uint64_t h, uint32_t cap, uint32_t hi) {
     return s < hi ? s : hi - 1u;
 }
 
+// Slots of a table that has to hold `cap` groups in np ranges.  Hashes spread
+// the groups over the ranges like balls over bins, so a range has its share,
+// six standard deviations of it and a few slots for the smallest shares; with
+// the share alone, which whole-table probing lives on, a table sized at two
+// slots a group overflowed for most key sets of 2049 groups in 256 ranges.
+inline uint64_t part_slots(uint64_t cap, uint32_t np) {
+    const double share = (double)cap / np;
+    return (uint64_t)np * (uint64_t)(share + 6.0 * std::sqrt(share) + 8.0);
+}
+
 // Key columns of a hashed group table are written by the lane that claims
 // a slot and compared by lanes on every XCD while the same kernel runs.
 // Plain stores would stay in the writer's L2, which the other XCDs do not
@@ -558,11 +570,11 @@ DQC_DEVICE_INLINE int lds_slot_exact(uint64_t* ltags, uint32_t cap, uint64_t tag
 }
 
 // Slot of `tag` in an LDS image of n group slots, probed from slot s on and
-// wrapping at n; -1 when LDS_IMAGE_PROBE slots hold other tags.
-constexpr uint32_t LDS_IMAGE_PROBE = 512;
-
-DQC_DEVICE_INLINE int lds_image_slot(uint64_t* itags, uint32_t n, uint64_t tag, uint32_t s) {
-    for (uint32_t k = 0; k < n && k < LDS_IMAGE_PROBE; ++k) {
+// wrapping at n; -1 when all hold other tags (or a table of the plan is known
+// to be too small: then the run is repeated, and long probes end).
+DQC_DEVICE_INLINE int lds_image_slot(uint64_t* itags, uint32_t n, uint64_t tag, uint32_t s, const uint32_t* status) {
+    for (uint32_t k = 0; k < n; ++k) {
+        if ((k & 31u) == 31u && overflow_raised(status)) return -1;
         const uint64_t t = __hip_atomic_load(&itags[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         if (t == tag) return (int)s;
         if (t == TAG_EMPTY) {

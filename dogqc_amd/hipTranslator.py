@@ -556,6 +556,9 @@ class Program(object):
         h.emit("    uint64_t cnt[%d];" % max(1, len(self.buffers)))
         h.emit("    uint64_t bytes;")
         h.emit("    int64_t htcap[%d];" % max(1, len(self.hts)))
+        padded = [r["index"] for r in self.hts if r.get("ranges")]
+        if padded:
+            h.emit("    int64_t htask[%d];     // slots asked for; htcap has room in every range" % len(self.hts))
         h.emit("    int64_t mment[%d];" % max(1, len(self.hts)))
         h.emit("    int64_t rcap;")
         h.emit("    int64_t tcap[%d];" % max(1, len(self.temps)))
@@ -667,6 +670,8 @@ class Program(object):
         h.emit("out->nhts = %d;" % len(self.hts))
         h.emit("for (int i = 0; i < %d; ++i) { out->ht_capacity[i] = L.htcap[i]; out->mm_entries[i] = L.mment[i]; "
                "out->split_capacity[i] = L.scap[i]; }" % len(self.hts))
+        for i in padded:
+            h.emit("out->ht_capacity[%d] = L.htask[%d];" % (i, i))
         h.emit("out->result_capacity = L.rcap;")
         res = self.result["columns"] if self.result else []
         h.emit("out->nresult = %d;" % len(res))
@@ -2124,8 +2129,9 @@ class AggregationTranslator(UnaryTranslator):
         aggregates there and writes the used slots back with plain stores:
         no claim and no atomic leaves the CU.  What PHASE 0 put into the
         range directly is read into the image first.  Every update of such a
-        table wraps its probes inside the range, and a full range reports an
-        overflow like a full table.  A range too large for LDS (beyond about
+        table wraps its probes inside the range, so the table gets more slots
+        than were asked for, enough that every range holds its groups when
+        the table was asked to (dqc::part_slots).  A range too large for LDS (beyond about
         8 M groups of one accumulator) is aggregated in an LDS table instead
         and flushed group by group, with slots over the whole table.
 
@@ -2155,7 +2161,8 @@ class AggregationTranslator(UnaryTranslator):
             f = "" if pipe.ldsFilter is None else " + " + pipe.ldsFilter["host"]
             return "(uint64_t)%du%s" % (staticLdsBytes(pipe) + 4 * (self.PART_MAX + self.PART_SEG_MAX + 1 + 17) + 1024, f)
         prog.hostVars["apart%d" % idx] = (
-            "{ const int32_t req = t->part_agg;\n"
+            "{ L.htask[%d] = L.htcap[%d];\n"
+            "  const int32_t req = t->part_agg;\n"
             "  const int64_t known = t->ht_capacity[%d] > 0 ? t->ht_capacity[%d] / 2 : %s;\n"
             "  uint32_t np = 0u;\n"
             "  if (req > 0) np = std::min<uint32_t>(%du, std::max<uint32_t>(2u, pow2floor((uint64_t)req)));\n"
@@ -2169,14 +2176,17 @@ class AggregationTranslator(UnaryTranslator):
             "    const double mu = (double)std::max<int64_t>(1, %s) / ((double)seg * np);\n"
             "    L.apseg[%d] = seg;\n"
             "    L.apcap[%d] = std::min<int64_t>(((int64_t)1 << 31) / seg, (int64_t)(mu * 1.25 + 4.0 * std::sqrt(mu)) + 16);\n"
-            "    const uint64_t span = (uint64_t)L.htcap[%d] / np + 1u;\n"
-            "    L.apimg[%d] = L.htcap[%d] >= (int64_t)np && span * %du + 256u + %s <= maxLds() ? (uint32_t)span : 0u;\n"
+            "    const uint64_t slots = dqc::part_slots((uint64_t)L.htcap[%d], np), span = slots / np;\n"
+            "    if (L.htcap[%d] >= (int64_t)np && slots < 0xffffffffull && span * %du + 256u + %s <= maxLds()) {\n"
+            "      L.apimg[%d] = (uint32_t)span; L.htcap[%d] = (int64_t)slots;\n"
+            "    }\n"
             "  } }"
-            % (idx, idx, groupsKnown, self.PART_MAX, cfgParts, cfgParts, self.PART_MIN_GROUPS,
+            % (idx, idx, idx, idx, groupsKnown, self.PART_MAX, cfgParts, cfgParts, self.PART_MIN_GROUPS,
                prog.estimate(a.child), self.PART_MIN_ROWS, self.PART_MAX, self.PART_AUTO_MIN, self.PART_GROUPS,
                idx, idx, idx, est,
                self.PART_SEG_MAX, pipe.pipeId, pipe.pipeId, pipe.defaultGrid, pipe.params["n"][1], B * U,
-               prog.estimate(a.child), idx, idx, idx, idx, idx, slotBytes, used()))
+               prog.estimate(a.child), idx, idx, idx, idx, slotBytes, used(), idx, idx))
+        self.ht["ranges"] = True
         # a record is 1 + (inputs) 8-byte words, stored row-wise so that a
         # partition's records in a segment share cache lines
         K = 1 + sum(1 for acc in self.accs if acc["kind"] != "count")
@@ -2267,7 +2277,7 @@ class AggregationTranslator(UnaryTranslator):
         with pipe.rowLoop():
             pipe.code.open("if (active[u])")
             pipe.emit("const uint64_t gh = dqc::mix64(%s);" % ptag)
-            pipe.emit("const int li = dqc::lds_image_slot(itags, ihi - ilo, %s, dqc::part_home(gh, %s, ihi) - ilo);"
+            pipe.emit("const int li = dqc::lds_image_slot(itags, ihi - ilo, %s, dqc::part_home(gh, %s, ihi) - ilo, &st->flags);"
                       % (ptag, upd["fcap"]))
             pipe.code.open("if (li >= 0)")
             for acc, v in zip(self.accs, vals1):
