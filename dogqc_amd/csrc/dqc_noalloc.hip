@@ -140,9 +140,10 @@ extern "C" int dqc_query_run_noalloc(void* module, const dqc_plan_inputs* in, dq
     if (rc) return rc;
 
     hipStream_t s = (hipStream_t)stream;
+    const dqcrt::KeepChoices keep(tun);
     for (int attempt = 0;; ++attempt) {
         dqc_plan_layout L;
-        rc = m->layout(in, tun, &L);
+        rc = dqcrt::layoutWithin(m, in, tun, (uint64_t)DQC_NOALLOC_WS_BYTES, &L);
         if (rc) return fail(rc, "plan layout failed (%d)", rc);
         if (L.ws_bytes > (uint64_t)DQC_NOALLOC_WS_BYTES)
             return fail(DQC_ENOMEM,

@@ -88,6 +88,18 @@ bool adjustForRetry(const dqc_plan_layout& L, const dqc_plan_status& st, dqc_pla
     return retry;
 }
 
+int layoutWithin(const Module* m, const dqc_plan_inputs* in, dqc_plan_tuning* tun, uint64_t limit,
+                 dqc_plan_layout* L) {
+    int rc = m->layout(in, tun, L);
+    for (int32_t* choice : {&tun->part_agg, &tun->join_filter}) {
+        if (rc || L->ws_bytes <= limit) return rc;
+        if (*choice != 0) continue;
+        *choice = -1;
+        rc = m->layout(in, tun, L);
+    }
+    return rc;
+}
+
 namespace {
 
 constexpr uint64_t WS_KEEP_BYTES = 2ull << 30;
@@ -371,6 +383,7 @@ int dqc_query_run(void* module, const dqc_plan_inputs* in, dqc_plan_tuning* tun,
     if (!module || !in || !tun || !res) return fail(DQC_EINVAL, "dqc_query_run: null argument");
     memset(res, 0, sizeof(*res));
     Module* m = (Module*)module;
+    const dqcrt::KeepChoices keep(tun);
     for (int attempt = 0;; ++attempt) {
         dqc_plan_layout L;
         int rc = m->layout(in, tun, &L);
@@ -380,6 +393,14 @@ int dqc_query_run(void* module, const dqc_plan_inputs* in, dqc_plan_tuning* tun,
             res->ws = nullptr;
             if (old && (rc = dqcrt::wsRelease(old)) != DQC_OK) return rc;
             rc = dqcrt::wsAcquire(&res->ws, L.ws_bytes);
+            while (rc == DQC_ENOMEM) {
+                // with less of what the plan can do without, if that is less
+                const uint64_t refused = L.ws_bytes;
+                const int lrc = dqcrt::layoutWithin(m, in, tun, refused - 1, &L);
+                if (lrc) return fail(lrc, "plan layout failed (%d)", lrc);
+                if (L.ws_bytes >= refused) break;
+                rc = dqcrt::wsAcquire(&res->ws, L.ws_bytes);
+            }
             if (rc) return rc;
             res->ws_bytes = L.ws_bytes;
         }

@@ -25,6 +25,23 @@ struct Module {
 // their exact counts).  Returns true when the run has to be repeated.
 bool adjustForRetry(const dqc_plan_layout& L, const dqc_plan_status& st, dqc_plan_tuning* tun);
 
+// The plan's layout, within `limit` bytes if it can be: a workspace too large
+// does without the memory that the plan takes only to be faster when the
+// tuning leaves the choice to it (the record segments of partitioned
+// group-bys, then join filters: part_agg and join_filter 0, set to -1 here).
+// The caller looks whether L->ws_bytes fits.
+int layoutWithin(const Module* m, const dqc_plan_inputs* in, dqc_plan_tuning* tun, uint64_t limit,
+                 dqc_plan_layout* L);
+
+// Sets the two fields layoutWithin may have changed back, so that a caller's
+// tuning keeps what it asked for.
+struct KeepChoices {
+    dqc_plan_tuning* tun;
+    int32_t part_agg, join_filter;
+    explicit KeepChoices(dqc_plan_tuning* t) : tun(t), part_agg(t->part_agg), join_filter(t->join_filter) {}
+    ~KeepChoices() { tun->part_agg = part_agg; tun->join_filter = join_filter; }
+};
+
 // Workspaces of dqc_query_run.  A workspace handed out is an allocation of
 // its own (hipMalloc); one that is released waits here for the next run that
 // fits it, because allocating and freeing costs more than most plans: 0.3 ms

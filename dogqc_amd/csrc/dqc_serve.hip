@@ -334,7 +334,7 @@ struct Server {
         // every (re)admission: what any query of the module needed so far
         if (cfg.size_feedback) applyFeedback(r);
         dqc_plan_layout L;
-        int rc = r.module->layout(&r.inputs, &r.tuning, &L);
+        int rc = dqcrt::layoutWithin(r.module, &r.inputs, &r.tuning, cfg.arena_bytes, &L);
         if (rc) {
             fail(rc, "plan layout failed (%d)", rc);
             finish(r, DQC_SERVE_FAILED, rc);

@@ -215,7 +215,9 @@ int dqc_query_release(dqc_query_result* res);
  * capture, tight serving loops, hosts that forbid hipMalloc).  The plan runs
  * in the library's static workspace; a plan whose workspace (the layout's
  * ws_bytes) exceeds DQC_NOALLOC_WS_BYTES, also after a retry enlarged its
- * tables, is rejected with DQC_ENOMEM.  The caller passes one device buffer
+ * tables, runs without the memory it takes only to be faster (what part_agg
+ * and join_filter left at 0 let it choose) and is rejected with DQC_ENOMEM
+ * if that is not enough.  The caller passes one device buffer
  * per result column (out_cols, in describe() order, each holding out_rows
  * rows of its column's type); the result rows are copied there and a result
  * of more than out_rows rows fails with DQC_EOVERFLOW.  res receives the

@@ -161,6 +161,42 @@ def test_admission_respects_arena_and_rejects_oversized():
     small.destroy()
 
 
+def test_arena_decides_over_a_plans_own_choices():
+    """A query whose partition records do not fit the arena runs without
+    them; one that asks for partitions fails as before."""
+    print("gpu case: serving without partitions", flush=True)
+    T = tables(0.02)
+    plans = serving.PlanSet(tuned=False)
+    rows = serving.prefixRows(T, "c3", 0.02)
+    mod, _ = plans.pick("c3", max(rows.values()))
+    r, cols = serving.binding(mod, T, rows)
+
+    class Bound(object):
+        struct = rt.Inputs(len(r), len(cols), r.ctypes.data_as(C.POINTER(C.c_int64)), C.cast(cols, C.POINTER(C.c_void_p)))
+
+    def tuning(parts):
+        t = rt.newTuning()
+        t.part_agg = parts
+        for h in mod.desc["hts"]:
+            if h["kind"] == "agg":
+                t.ht_capacity[h["index"]] = 100000
+        return t
+    lean, full = [int(rt.layout(mod, Bound, tuning(p)).ws_bytes) for p in (-1, 0)]
+    asked = int(rt.layout(mod, Bound, tuning(256)).ws_bytes)
+    assert lean < full <= asked
+    for parts, arena, state in ((0, lean, 2), (0, full, 2), (256, lean, 3)):
+        srv = serving.Server(2, arena)
+        qid = srv.submit(mod, r, cols, tuning(parts), keep=True)
+        srv.start()
+        srv.wait(60000)
+        rec = srv.record(qid)
+        assert rec.state == state and rec.retries == 0, (parts, arena)
+        if state == 2:
+            got = serving.resultOf(plans, "c3", rec)
+            assert servecheck.matchesOracle("c3", got, servecheck.oracleResult(T, "c3", 0.02))
+        srv.destroy()
+
+
 def test_overflow_is_readmitted():
     print("gpu case: serving retry", flush=True)
     T = tables(0.02)

@@ -136,3 +136,37 @@ def test_noalloc_rejects_oversized_workspace_and_short_outputs():
     oracle, tol = oracleOf("c1", acc)
     assertSameResult(got, want, tol, label="c1 after the refusals")
     assertSameResult(got, oracle, tol, label="c1 after the refusals vs oracle")
+
+
+def test_noalloc_partitions_only_where_they_fit():
+    """A group-by that partitions by itself, with record segments beyond the
+    static scratch, runs unpartitioned there; partitions asked for are not
+    dropped."""
+    n, keys = 3000000, 3000
+    acc = planlib.featureData(10, 10)
+    rng = np.random.default_rng(5)
+    for name in ("t_id", "t_grp", "t_cat", "t_val", "t_f", "t_big", "t_date"):
+        col = np.asarray(acc.column("t", name))
+        acc.data[("t", name)] = np.resize(col, n)
+    acc.data[("t", "t_big")] = (np.arange(n, dtype=np.int64) % keys) << 30
+    acc.data[("t", "t_f")] = rng.integers(0, 100, n).astype(np.float32)
+    acc.schema["t"]["size"] = n
+    mod = module("f_groupby_int64")
+    inputs = rt.BoundInputs(mod, acc)
+
+    def tuning(parts):
+        t = rt.newTuning()
+        t.part_agg, t.ht_capacity[0], t.result_capacity = parts, 2 * keys, keys
+        return t
+    assert rt.layout(mod, inputs, tuning(0)).ws_bytes > rt.NOALLOC_WS_BYTES > rt.layout(mod, inputs, tuning(-1)).ws_bytes
+    print("gpu case: noalloc f_groupby_int64, segments beyond the scratch", flush=True)
+    t = tuning(0)
+    got, res = noallocColumns(mod, inputs, acc, keys, t)
+    assert res.retries == 0 and t.part_agg == 0
+    want = np.bincount(np.arange(n) % keys, weights=np.asarray(acc.column("t", "t_f")).astype(np.float64))
+    order = np.argsort(got["t_bq"])
+    assert np.array_equal(got["t_bq"][order], np.arange(keys))
+    assert np.array_equal(got["sf"][order], want)           # whole numbers: exact in any order
+    assert (got["c"] == n // keys).all()
+    with pytest.raises(rt.DqcError, match="static scratch"):
+        noallocColumns(mod, inputs, acc, keys, tuning(256))
