@@ -79,7 +79,9 @@ class EquiJoinTranslator(BinaryTranslator):
     SPLIT_CHUNK = 16
     DEFAULT_SPLIT_THRESHOLD = 1024   # list length above which a probe row is queued
     # unique inner joins at most this selective can take a filter of their
-    # build keys (tuning join_filter = n KB, up to 4 MB; off by default): in
+    # build keys (tuning join_filter = n KB, up to 4 MB; with 0 the plan's
+    # default below, else 16 bits a key in device memory where a lane refill
+    # gathers the rows that pass, see _refillBeforeProbe, else none): in
     # LDS when it fits beside the probe pipeline's other LDS (every workgroup
     # copies it, so it pays with few, large workgroups; the autotuner
     # searches size and grid together), else probed in device memory, where
@@ -270,6 +272,7 @@ class EquiJoinTranslator(BinaryTranslator):
             # (defaultJoinFilter, none unless a plan is translated with one)
             req = "t->join_filter" if not EquiJoinTranslator.defaultJoinFilter else \
                 "(t->join_filter != 0 ? t->join_filter : %d)" % int(EquiJoinTranslator.defaultJoinFilter)
+            ht["filterReq"] = req
             # (a join whose refill stands before its probe: 16 bits a key, in
             # device memory)
             auto = ""
@@ -944,11 +947,12 @@ class EquiJoinTranslator(BinaryTranslator):
         J = self.algExpr.opId
         prog = ctxt.program
         pid = pipe.pipeId
-        # words in this pipeline: the build's, if they fit with the static LDS
+        # words in this pipeline: the build's, if a size was asked for (by the
+        # tuning or as the plan's default) and they fit with the static LDS
         # and 16 KB to spare for an LDS group table
         prog.hostVars["bfp%d" % pid] = lambda: (
-            "L.bfp[%d] = t->join_filter > 0 && (uint64_t)L.bfw[%d] * 4u + %du + 16384u <= maxLds() ? L.bfw[%d] : 0u;"
-            % (pid, idx, staticLdsBytes(pipe) + 1024, idx))
+            "L.bfp[%d] = %s > 0 && (uint64_t)L.bfw[%d] * 4u + %du + 16384u <= maxLds() ? L.bfw[%d] : 0u;"
+            % (pid, self.ht["filterReq"], idx, staticLdsBytes(pipe) + 1024, idx))
         fbf = pipe.param("jbf%d" % J, "const uint32_t*", "B_jbf%d" % J)
         pipe.param("jbfp%d" % J, "uint32_t", "L.bfp[%d]" % pid)
         pipe.param("jbfg%d" % J, "uint32_t", "L.bfp[%d] ? 0u : L.bfw[%d]" % (pid, idx))

@@ -93,9 +93,10 @@ typedef struct dqc_plan_tuning {
                                                 exceeds 2048 and the input 65536 rows, -1 = never,
                                                 n > 0 = n partitions */
     int32_t join_filter;                     /* filter of the build keys of selective unique joins: n > 0 =
-                                                n KB (in LDS when it fits), 0 = 16 bits per key in device
-                                                memory for a join whose lane refill gathers the rows that
-                                                pass it, else the plan's default; < 0 = none */
+                                                n KB (in LDS when it fits), 0 = the size the plan was
+                                                translated with, else 16 bits per key in device memory for
+                                                a join whose lane refill gathers the rows that pass it,
+                                                else none; < 0 = none */
     int32_t part_build;                      /* partitioned unique-join build (plans translated with it):
                                                 n > 0 = n partitions, else none */
     int32_t reserved[2];

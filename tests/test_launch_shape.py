@@ -112,6 +112,40 @@ def test_refill_front(plan, n):
         check(plan, acc, tuning=t, label="n=%d grid=%d threshold=%d filter=%d" % (n, grid, threshold, jf))
 
 
+def test_default_filter_is_held_in_lds(tmp_path):
+    """A filter of a size the plan was translated with goes to LDS like one
+    the tuning asks for; the size chosen from the key count does not.  (The
+    generated host code's own statements, compiled for the host.)"""
+    import re
+    import subprocess
+
+    def words(default, request):
+        alg, p, cfg, opts = planlib.build("c3_refill", planlib.emptyAccessor("c3_refill"))
+        plan = alg.resolveAlgebraPlan(p, cfg)
+        with planlib.knobs(joinFilter=default):
+            comp = planlib.HipCompiler(alg, "gfx950", planlib.CType.FP64)
+            comp.setBuffers(opts["buffers"])
+            comp.gencode(alg.translateToCompilerPlan(plan, comp))
+        size = re.search(r"\{ const int32_t req = .*?L\.bfw\[2\] = w; \}", comp.source, re.S).group(0)
+        held = re.search(r"L\.bfp\[\d+\] = [^;]*\? L\.bfw\[2\] : 0u;", comp.source).group(0)
+        helpers = "".join(re.search(r"static inline uint32_t pow2%s\(.*\n" % f, comp.source).group(0)
+                          for f in ("floor", "ceil"))
+        (tmp_path / "w.cpp").write_text(
+            "#include <algorithm>\n#include <cstdint>\n#include <cstdio>\n" + helpers +
+            "static uint64_t maxLds() { return 163840; }\n"
+            "int main() { struct { uint32_t bfw[4], bfp[4]; int64_t htcap[4]; } L = {}; L.htcap[2] = 60000;\n"
+            "struct { int32_t join_filter; } T = {%d}, *t = &T;\n%s\n%s\n"
+            "printf(\"%%u %%u\\n\", L.bfw[2], L.bfp[0] + L.bfp[1] + L.bfp[2] + L.bfp[3]); }\n" % (request, size, held))
+        subprocess.run(["g++", "-std=c++17", "-w", str(tmp_path / "w.cpp"), "-o", str(tmp_path / "w")], check=True)
+        return [int(x) for x in subprocess.run([str(tmp_path / "w")], stdout=subprocess.PIPE, check=True).stdout.split()]
+
+    assert words(32, 0) == words(0, 32) == [8192, 8192]
+    assert words(32, -1) == words(0, -1) == [0, 0]
+    assert words(32, 64) == [16384, 16384]
+    assert words(0, 0) == [16384, 0]
+    assert words(2048, 0) == [524288, 0]
+
+
 @pytest.mark.parametrize("plan", ["c2_pushdown", "c2_both", "c3_refill", "f_like_project_refill", "tpch3", "tpch5",
                                   "tpch7", "tpch8", "tpch9", "tpch10", "tpch14", "tpch19"])
 @pytest.mark.parametrize("budget", [80 << 10, 40 << 10, 16 << 10, 0])
