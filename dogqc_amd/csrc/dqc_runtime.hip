@@ -20,6 +20,7 @@
 #include <cstdio>
 #include <cstring>
 #include <mutex>
+#include <new>
 #include <string>
 #include <unordered_map>
 #include <vector>
@@ -105,6 +106,8 @@ namespace {
 constexpr uint64_t WS_KEEP_BYTES = 2ull << 30;
 constexpr size_t WS_KEEP_BLOCKS = 16;
 constexpr uint64_t WS_KEEP_ACQUIRES = 256;
+// a run takes a waiting block of at most this many times its size and 4 MB
+constexpr uint64_t WS_FIT_FACTOR = 2, WS_FIT_BYTES = 4ull << 20;
 
 struct WsBlock {
     void* ptr;
@@ -144,19 +147,24 @@ int wsAcquire(void** ptr, uint64_t bytes) {
     if (bytes == 0) bytes = 256;
     int device = 0;
     HIP_CHECK(hipGetDevice(&device), "hipGetDevice");
+    const uint64_t most = WS_FIT_FACTOR * bytes + WS_FIT_BYTES;
     WsPool& p = pool();
     {
         std::lock_guard<std::mutex> g(p.lock);
         ++p.acquires;
         size_t best = p.free.size();
         for (size_t i = 0; i < p.free.size(); ++i)
-            if (p.free[i].device == device && p.free[i].bytes >= bytes &&
+            if (p.free[i].device == device && p.free[i].bytes >= bytes && p.free[i].bytes <= most &&
                 (best == p.free.size() || p.free[i].bytes < p.free[best].bytes))
                 best = i;
         if (best < p.free.size()) {
             const WsBlock b = p.free[best];
+            try {
+                p.out[b.ptr] = b;
+            } catch (const std::bad_alloc&) {
+                return fail(DQC_ENOMEM, "workspace list: out of host memory");
+            }
             p.free.erase(p.free.begin() + (long)best);
-            p.out[b.ptr] = b;
             *ptr = b.ptr;
             return DQC_OK;
         }
@@ -164,7 +172,11 @@ int wsAcquire(void** ptr, uint64_t bytes) {
     const int rc = dqc_malloc(ptr, bytes);
     if (rc) return rc;
     std::lock_guard<std::mutex> g(p.lock);
-    p.out[*ptr] = WsBlock{*ptr, bytes, device, 0};
+    try {
+        p.out[*ptr] = WsBlock{*ptr, bytes, device, 0};
+    } catch (const std::bad_alloc&) {
+        // not in the list: freed at its release
+    }
     return DQC_OK;
 }
 
@@ -187,21 +199,28 @@ int wsRelease(void* ptr) {
         HIP_CHECK(hipFree(ptr), "hipFree");
         return DQC_OK;
     }
-    std::vector<void*> drop;
+    // as many blocks leave as have to for this one to wait (at most all of
+    // them: WS_KEEP_BLOCKS + 1 with it)
+    void* drop[WS_KEEP_BLOCKS + 1];
+    size_t ndrop = 0;
     {
         std::lock_guard<std::mutex> g(p.lock);
         b.since = p.acquires;
-        p.free.push_back(b);
         uint64_t kept = 0;
+        try {
+            p.free.push_back(b);
+        } catch (const std::bad_alloc&) {
+            drop[ndrop++] = b.ptr;
+        }
         for (const WsBlock& f : p.free) kept += f.bytes;
-        while (kept > WS_KEEP_BYTES || p.free.size() > WS_KEEP_BLOCKS ||
-               p.acquires - p.free.front().since > WS_KEEP_ACQUIRES) {
+        while (!p.free.empty() && (kept > WS_KEEP_BYTES || p.free.size() > WS_KEEP_BLOCKS ||
+                                   p.acquires - p.free.front().since > WS_KEEP_ACQUIRES)) {
             kept -= p.free.front().bytes;
-            drop.push_back(p.free.front().ptr);
+            drop[ndrop++] = p.free.front().ptr;
             p.free.erase(p.free.begin());
         }
     }
-    for (void* d : drop) (void)hipFree(d);
+    for (size_t i = 0; i < ndrop; ++i) (void)hipFree(drop[i]);
     return DQC_OK;
 }
 
@@ -425,6 +444,11 @@ int dqc_query_release(dqc_query_result* res) {
     res->ws = nullptr;
     res->ws_bytes = 0;
     return rc;
+}
+
+int dqc_workspace_trim(void) {
+    dqcrt::wsTrim();
+    return DQC_OK;
 }
 
 int dqc_graph_create(void* module, const dqc_plan_inputs* in, const dqc_plan_tuning* tun, void* ws,

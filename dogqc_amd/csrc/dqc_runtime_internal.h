@@ -48,10 +48,12 @@ struct KeepChoices {
 // for 100 MB and more, and 8 ms where the process holds gigabytes (a TPC-H Q18
 // call at SF1 9.0 ms, 0.34 ms with waiting workspaces).
 //   * bounded: at most 2 GiB and 16 blocks wait, the oldest are freed first;
-//     a larger workspace is freed at once;
+//     a larger workspace is freed at once; a run takes no block of more than
+//     twice its size and 4 MB, so a small result that is kept holds no large one;
 //   * given back: blocks no run has asked for in 256 acquisitions are freed,
-//     all when an allocation of this library fails and when the last plan
-//     module is unloaded;
+//     all when an allocation of this library fails, when the last plan
+//     module is unloaded and when the program asks (dqc_workspace_trim), for
+//     instance before another allocator of the process needs the memory;
 //   * released like hipFree: the device's pending work is waited for, so work
 //     on any stream that still reads the results has ended before the memory
 //     is handed out again;

@@ -26,6 +26,7 @@ RUNTIME_SYMBOLS = [
     "dqc_query_release", "dqc_graph_create", "dqc_graph_launch", "dqc_graph_destroy",
     "dqc_serve_create", "dqc_serve_submit", "dqc_serve_start", "dqc_serve_wait", "dqc_serve_record_of",
     "dqc_serve_release", "dqc_serve_destroy", "dqc_query_run_noalloc",
+    "dqc_workspace_trim",
 ]
 NOALLOC_WS_BYTES = 64 << 20  # DQC_NOALLOC_WS_BYTES
 GEN_SYMBOLS = ["dqc_gen_uniform", "dqc_gen_decimal", "dqc_gen_pick_u32", "dqc_gen_affine_perm",
@@ -529,6 +530,12 @@ def run(module, inputs, tuning=None, stream=None, max_retries=8, feedback=None):
     if feedback is not None:
         feedback.learn(module, inputs, ex)
     return ex
+
+
+def trimWorkspaces():
+    """Free the released workspaces that wait for later runs (up to 2 GiB),
+    for instance before another allocator of the process needs the memory."""
+    check(lib().dqc_workspace_trim(), "dqc_workspace_trim")
 
 
 def runNoAlloc(module, inputs, outputs, out_rows, tuning=None, stream=None, max_retries=8):

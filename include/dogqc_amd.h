@@ -198,13 +198,15 @@ typedef struct dqc_query_result {
     int32_t retries;
 } dqc_query_result;
 
-/* Run a plan to completion on `stream`: allocate the workspace (a released
- * one of about the size if there is one, dqc_query_release), enqueue,
- * synchronise, and on a full hash table, multimap, temp table or result buffer enlarge
+/* Run a plan to completion on `stream`: allocate the workspace (or take a
+ * released one, of at most twice the size and 4 MB), enqueue, synchronise, and on a full hash table, multimap, temp table or result buffer enlarge
  * it (tuning is updated in place) and run again, up to max_retries times. */
 int dqc_query_run(void* module, const dqc_plan_inputs* in, dqc_plan_tuning* tun, void* stream,
                   int32_t max_retries, dqc_query_result* res);
+/* Give a result's workspace back.  Up to 2 GiB of released workspaces wait in
+ * the library for later runs; dqc_workspace_trim frees them all. */
 int dqc_query_release(dqc_query_result* res);
+int dqc_workspace_trim(void);
 
 /* Workspace size of dqc_query_run_noalloc: a static device array compiled
  * into libdqcrt.so, one copy per GPU the library runs on, held until the

@@ -47,6 +47,43 @@ def test_a_larger_run_after_a_smaller():
         ex.release()
 
 
+def test_a_kept_small_result_leaves_the_large_block():
+    small, large = start("c1", {"dim": 50, "fact": 100}, 6), start("c1", {"dim": 2400000, "fact": 1000}, 7)
+    rt.trimWorkspaces()
+    ex = rt.run(large[1], large[2])
+    block = ex.res.ws
+    assert ex.res.ws_bytes > (5 << 20)
+    ex.release()
+    kept = rt.run(small[1], small[2])
+    assert kept.res.ws != block
+    ex = rt.run(large[1], large[2])
+    assert ex.res.ws == block
+    verify(large[0], large[1], ex, large[3], "large again")
+    ex.release()
+    verify(small[0], small[1], kept, small[3], "kept small")
+    kept.release()
+
+
+def freeBytes():
+    free, total = rt.C.c_size_t(), rt.C.c_size_t()
+    assert rt.lib().hipMemGetInfo(rt.C.byref(free), rt.C.byref(total)) == 0
+    return free.value
+
+
+def test_trim_gives_the_memory_back():
+    job = start("c0", {"cfg0": 1000}, 8)
+    t = rt.newTuning()
+    t.result_capacity = 8 << 20         # some 700 MB of result columns
+    before = freeBytes()
+    ex = rt.run(job[1], job[2], t)
+    size = ex.res.ws_bytes
+    verify(job[0], job[1], ex, job[3], "large result")
+    ex.release()
+    assert before - freeBytes() >= size // 2
+    rt.trimWorkspaces()
+    assert before - freeBytes() < size // 2
+
+
 def test_threads():
     jobs = [start("c1", {"dim": 1000 * (k + 1), "fact": 30000}, 10 + k) for k in range(4)]
     failures = []
