@@ -142,6 +142,12 @@ void wsTrim() {
     for (const WsBlock& b : all) (void)hipFree(b.ptr);
 }
 
+void wsForget(void* ptr) {
+    WsPool& p = pool();
+    std::lock_guard<std::mutex> g(p.lock);
+    p.out.erase(ptr);
+}
+
 int wsAcquire(void** ptr, uint64_t bytes) {
     *ptr = nullptr;
     if (bytes == 0) bytes = 256;
@@ -262,6 +268,8 @@ int dqc_malloc(void** ptr, uint64_t bytes) {
 }
 
 int dqc_free(void* ptr) {
+    // (a workspace freed here is none any more: another allocation may get its address)
+    if (ptr) dqcrt::wsForget(ptr);
     if (ptr) HIP_CHECK(hipFree(ptr), "hipFree");
     return DQC_OK;
 }

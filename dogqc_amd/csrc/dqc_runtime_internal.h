@@ -62,6 +62,7 @@ struct KeepChoices {
 int wsAcquire(void** ptr, uint64_t bytes);
 int wsRelease(void* ptr);
 void wsTrim();
+void wsForget(void* ptr);
 
 }  // namespace dqcrt
 

@@ -84,6 +84,24 @@ def test_trim_gives_the_memory_back():
     assert before - freeBytes() < size // 2
 
 
+def test_a_workspace_freed_by_hand_is_forgotten():
+    """dqc_free on a result's workspace, as dqc_query_release did at first:
+    a smaller allocation that gets the address is not taken for it."""
+    job = start("c1", {"dim": 600000, "fact": 1000}, 9)
+    rt.trimWorkspaces()
+    ex = rt.run(job[1], job[2])
+    rt.check(rt.lib().dqc_free(ex.res.ws), "dqc_free")
+    ex.res.ws = None
+    other = rt.DeviceBuffer(4096)
+    res = rt.QueryResult()
+    res.ws, res.ws_bytes = other.ptr.value, 4096
+    rt.check(rt.lib().dqc_query_release(rt.C.byref(res)), "dqc_query_release")
+    other.ptr = rt.C.c_void_p()
+    ex = rt.run(job[1], job[2])
+    verify(job[0], job[1], ex, job[3], "after dqc_free")
+    ex.release()
+
+
 def test_threads():
     jobs = [start("c1", {"dim": 1000 * (k + 1), "fact": 30000}, 10 + k) for k in range(4)]
     failures = []
