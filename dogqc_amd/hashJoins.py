@@ -151,11 +151,23 @@ class EquiJoinTranslator(BinaryTranslator):
         whole wavefronts, runs on dense lanes (c3's sales kernel with the
         refill after the probe 763 us, with a 256 KB filter 706 us, with the
         refill between the two 625 us).  Such a join has its filter unless
-        the tuning turns it off (join_filter < 0)."""
+        the tuning turns it off (join_filter < 0).  (The queue then holds the
+        probe keys, and the refill stays above the probe where LDS is short.)"""
         from dogqc_amd.hipDivergenceBuffer import LaneRefill, BufferType
         r = self.parent
         return r if self.filtered and isinstance(r, LaneRefill) and r.bufferType is BufferType.SMEM and \
             r.algExpr is self.algExpr else None
+
+    def _queueBefore(self, pipe, keep):
+        """The refill's queue before the probe, of the registers that carry
+        `keep`, fits LDS, or is no larger than after it: there it holds the
+        slot instead of the probe keys."""
+        from dogqc_amd.hipTranslator import pipelineSource, queueOfFits, registersBytes
+        out = self.algExpr.outRelation
+        live = pipe.liveState(keep)
+        after = pipe.liveState([att for id, att in out.items() if id in self.rightChild.algExpr.outRelation])
+        slot = 8 if any(id in self.leftChild.algExpr.outRelation for id in out) else 0
+        return registersBytes(live) <= registersBytes(after) + slot or queueOfFits(pipe, live, pipelineSource(self))
 
     def _preHash(self, pipe):
         """Wavefront string hashes of the probe keys (StringHash.wave), at
@@ -798,14 +810,15 @@ class EquiJoinTranslator(BinaryTranslator):
                       "dqc::bloom_test(p.jbf%d, p.jbfg%d, jh%d))" % (J, lbf, J, J, J, J, J)) \
                 if lbf is not None else None
             refill = self._refillBeforeProbe() if lbf is not None else None
-            if refill is not None and refill.possible(ctxt):
+            keep = [att for id, att in a.outRelation.items() if id in self.rightChild.algExpr.outRelation] + \
+                self.probeKeys + condProbe
+            if refill is not None and refill.possible(ctxt) and self._queueBefore(pipe, keep):
                 with pipe.rowLoop():
                     pipe.code.open("if (active[u])")
                     self._hashCode(pipe, self.probeKeys, jtag, "jh%d" % J, tagIsReg=True)
                     pipe.emit("active[u] = (p.jbfp%d == 0u && p.jbfg%d == 0u) || %s;" % (J, J, passes))
                     pipe.code.close()
-                keep = [att for id, att in a.outRelation.items() if id in self.rightChild.algExpr.outRelation]
-                refill.refill(ctxt, keep + self.probeKeys + condProbe,
+                refill.refill(ctxt, keep,
                               lambda c: self._probeUnique(c, pipe, None, refill.parent))
                 return
             self._probeUnique(ctxt, pipe, passes, self.parent)

@@ -1132,12 +1132,49 @@ def rowsPerThread(translator):
     # loads are in flight together, and the queue takes them one after
     # another); above it, and with any other loop, it is one row per lane.
     # (Q10's lineitem kernel 247 -> 221 us with four, c2's count pass 124 -> 97.)
-    # A row of the queue holds at most queuedBytes, and a wavefront
-    # 64 rows and 64 more per row that a thread carries.
     if not (_refillFirst(translator) or gatheringProbe(translator) is not None):
         return 1
-    rowBytes = (int(KernelCall.defaultBlockSize) // WAVE) * WAVE * queuedBytes(translator)
-    return max(1, min(U, FRONT_ROWS, QUEUE_LDS // rowBytes - 1))
+    return max(1, min(U, FRONT_ROWS, queueRows(translator)))
+
+
+def _queueRowBytes(translator):
+    return (int(KernelCall.defaultBlockSize) // WAVE) * WAVE * queuedBytes(translator)
+
+
+def queueRows(translator):
+    """Rows per thread that the pipeline's first queue has LDS for: it holds
+    at most queuedBytes a row, and for a wavefront 64 rows and 64 more per row
+    that a thread carries."""
+    return min(QUEUE_LDS, MAX_LDS - ldsAboveQueue(translator)) // _queueRowBytes(translator) - 1
+
+
+def queueFits(translator):
+    """The pipeline's first queue fits at one row per thread."""
+    return 2 * _queueRowBytes(translator) + ldsAboveQueue(translator) <= MAX_LDS
+
+
+def registersBytes(live):
+    """Bytes of a queue's row of these registers (Pipeline.liveState)."""
+    return sum(CType.size.get(ct, 8) for ct in live.values())
+
+
+def queueOfFits(pipe, live, translator):
+    """A first queue of the live registers, and the row index that goes with
+    them, fits the pipeline's LDS."""
+    row = 8 + registersBytes(live)
+    return staticLdsBytes(pipe) + pipe.bs * (pipe.U + 1) * row + ldsAboveQueue(translator) <= MAX_LDS
+
+
+def pipelineSource(translator):
+    """The operator that feeds the pipeline a translator consumes in."""
+    t = translator
+    while not isinstance(t, (LiteralTranslator, AggregationTranslator)):
+        t = t.rightChild if isinstance(t, BinaryTranslator) else t.child
+    return t
+
+
+def _registerBytes(a):
+    return 16 if a.dataType == Type.STRING else COLUMN_BYTES.get(a.dataType, 8)
 
 
 def queuedBytes(translator):
@@ -1146,7 +1183,6 @@ def queuedBytes(translator):
     and the row and slot indices of those not loaded yet."""
     from dogqc_amd.hashJoins import EquiJoinTranslator
     from dogqc_amd.hipDivergenceBuffer import LaneRefill
-    size = lambda a: 16 if a.dataType == Type.STRING else COLUMN_BYTES.get(a.dataType, 8)
     attrs, t, indices = {}, translator, 8
     while t is not None and not isinstance(t, LaneRefill):
         out = t.algExpr.outRelation
@@ -1162,11 +1198,42 @@ def queuedBytes(translator):
         if isinstance(t, EquiJoinTranslator) and t.algExpr.multimatch:
             break
         t = t.parent
-    return indices + sum(size(a) for a in attrs.values())
+    return indices + sum(_registerBytes(a) for a in attrs.values())
 
 
-# LDS that the queues of a workgroup with several rows per thread may take: two
-# such workgroups fit a CU (160 KB)
+def ldsAboveQueue(translator):
+    """At most the static LDS of a pipeline's operators above its first
+    queue: further queues, the scan of a push-down probe, the stage of a
+    materialisation, and what belongs to no row."""
+    from dogqc_amd.hashJoins import EquiJoinTranslator
+    from dogqc_amd.hipDivergenceBuffer import LaneRefill
+    nw = int(KernelCall.defaultBlockSize) // WAVE
+    total, queues, attrs, indices, t = 1024, 0, dict(translator.algExpr.outRelation), 8, translator
+    while t.parent is not None:
+        p = t.parent
+        if isinstance(p, EquiJoinTranslator):
+            indices += 8 + 8 + 4 + 4
+            attrs.update(p.algExpr.leftChild.outRelation)
+            if p.algExpr.multimatch:
+                total += nw * WAVE * 8
+        attrs.update(p.algExpr.outRelation)
+        row = indices + sum(_registerBytes(a) for a in attrs.values())
+        if isinstance(p, LaneRefill):
+            queues += 1
+            total += nw * WAVE * 2 * row if queues > 1 else 0
+        if isinstance(p, AggregationTranslator) or (isinstance(p, BinaryTranslator) and p.leftChild is t):
+            break
+        if isinstance(p, MaterializeTranslator):
+            out = sum(_registerBytes(a) for a in p.algExpr.outRelation.values())
+            total += nw * max(MaterializeTranslator.STAGE_BYTES_PER_WAVE, WAVE * out)
+            break
+        t = p
+    return total
+
+
+# LDS of a CU, and what the first queue of a workgroup with several rows per
+# thread may take of it: two such workgroups fit a CU
+MAX_LDS = 160 << 10
 QUEUE_LDS = 80 << 10
 FRONT_ROWS = 4
 # rows per wavefront of a pipeline with a lane refill: in one round of
@@ -1194,7 +1261,7 @@ def gatheringProbe(translator):
             fraction *= float(getattr(p.algExpr, "selectivity", 1.0))
         elif isinstance(p, EquiJoinTranslator):
             if p.algExpr.multimatch and p.algExpr.joinType in (Join.INNER, Join.OUTER):
-                return p if p.gathers(fraction) else None
+                return p if p.gathers(fraction) and queueFits(translator) else None
             if p.algExpr.joinType in (Join.INNER, Join.SEMI):
                 fraction *= min(1.0, float(getattr(p.algExpr, "selectivity", 1.0)))
         t = p

@@ -4,7 +4,10 @@ of the whole grid, and both have to reach every row exactly once."""
 import numpy as np
 import pytest
 
+import dogqc_amd.scalarAlgebra as scal
 from dogqc_amd import planlib, runtime as rt
+from dogqc_amd.relationalAlgebra import Reduction
+from dogqc_amd.types import Type
 from tests.test_gpu_parity import check, workloadAcc
 
 GRID = 3
@@ -163,6 +166,54 @@ def test_queue_stays_in_its_lds(plan, budget, monkeypatch):
         rows = (pipe.bs // 64) * 64 * (pipe.frontU + 1)
         assert H.staticLdsBytes(pipe) <= rows * sum(bounds), (plan, bounds)
         assert pipe.frontU == 1 or rows * max(bounds) <= budget
+
+
+def _twoRefills(alg, A, C):
+    """A group table through two lane refills into a result of 20 bytes a row."""
+    p = alg.projection(["t_id", "g", "m"],
+                       alg.map("m", scal.MulExpr(A("g"), C("2", Type.DOUBLE)),
+                               alg.aggregation(["t_id"], [(Reduction.MIN, "t_val", "g")], alg.scan("t"))))
+    return p, {}, [2, 4]
+
+
+def _stringJoin(alg, A, C):
+    """A selective unique join on a string, a refill right above it and one
+    more below the result: the first queue before the probe would hold the key."""
+    p = alg.projection(["u_id", "u_w", "u_grp"],
+                       alg.selection(scal.LargerExpr(A("u_w"), C("1.5", Type.DOUBLE)),
+                                     alg.selection(scal.LargerExpr(A("u_grp"), C("2", Type.INT)),
+                                                   alg.join(("u_name", "t_txt"), alg.scan("u"), alg.scan("t")))))
+    return p, {3: {"multimatch": False, "selectivity": 0.1}}, [3, 5]
+
+
+def _wideProbe(alg, A, C):
+    """A push-down probe that few rows reach, of rows with many strings: it
+    gathers them where their queue fits."""
+    node, cols = alg.scan("t"), ["s%d" % k for k in range(8)]
+    for k, c in enumerate(cols):
+        node = alg.map(c, scal.SubstringExpr(A("t_txt"), C(str(k + 1), Type.INT), C("3", Type.INT)), node)
+    node = alg.selection(scal.LargerExpr(A("t_id"), C("2", Type.INT)), node)
+    node = alg.join(("u_grp", "t_grp"), alg.scan("u"), node)
+    for a, b in zip(cols, cols[1:]):
+        node = alg.selection(scal.NotExpr(scal.EqualsExpr(A(a), A(b))), node)
+    return alg.projection(["u_id", "s0"], node), {10: {"selectivity": 0.1}, 12: {"multimatch": True}}, []
+
+
+@pytest.mark.parametrize("plan", [_twoRefills, _stringJoin, _wideProbe])
+@pytest.mark.parametrize("block,rows", [(256, 4), (256, 8), (512, 4), (1024, 1), (1024, 4)])
+def test_queues_leave_lds_to_the_operators_above(plan, block, rows):
+    """All of a pipeline's static LDS fits a CU: the rows per thread, and the
+    place of a refill at a filtered join, leave room for what follows."""
+    from dogqc_amd import hipTranslator as H
+    alg = planlib.RelationalAlgebra(planlib.featureEmpty())
+    p, cfg, buffers = plan(alg, planlib._A, planlib._C)
+    resolved = alg.resolveAlgebraPlan(p, cfg)
+    with planlib.knobs(block=block, rowsPerThread=rows, pushdown=plan is _wideProbe):
+        comp = H.HipCompiler(alg, "gfx950", planlib.CType.FP64)
+        comp.setBuffers(buffers)
+        comp.gencode(alg.translateToCompilerPlan(resolved, comp))
+    assert block > 256 or any(q.refillPoints or q.drains for q in comp.program.pipes)
+    assert max(H.staticLdsBytes(q) for q in comp.program.pipes) <= 160 << 10
 
 
 def test_join_builds_take_a_row_per_thread():
