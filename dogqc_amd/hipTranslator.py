@@ -290,9 +290,14 @@ class Pipeline(object):
         # handler reserves, of 800) and 7 of up to 96: with large workgroups that
         # is one workgroup in two.  Q15's lineitem kernel at 1024 threads, 42
         # vector and 87 scalar registers, 40.5 us without the limit, 29.2 with
-        # it; c3's by-item aggregation 64.5 -> 52.9.  Not where one workgroup
-        # per CU runs anyway: there it only spills (TPC-H Q1 269 -> 276 us).
-        sgprs = " __attribute__((amdgpu_num_sgpr(80)))" if B >= 512 and not self.fewGroups else ""
+        # it; 20 M rows into 1 M groups, the second launch 266 -> 191.  Where one
+        # workgroup per CU runs anyway it only spills (TPC-H Q1 269 -> 276 us):
+        # not with few groups or more than half a CU's static LDS.  What the
+        # translator does not know stays limited and costs little: a group
+        # image of more than half a CU's LDS (3 M groups 268 -> 274 us), more
+        # than 64 vector registers (Q10's lineitem kernel at 106: 86.6 -> 87.1).
+        alone = self.fewGroups or staticLdsBytes(self) > MAX_LDS // 2
+        sgprs = " __attribute__((amdgpu_num_sgpr(80)))" if B >= 512 and not alone else ""
         k.open("__global__ void __launch_bounds__(%d)%s %s(const KP_%s p)" % (B, sgprs, self.name, self.name))
         for d in self.staticLds:
             k.emit(d)

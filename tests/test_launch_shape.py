@@ -232,7 +232,15 @@ def test_join_build_grid(n):
 
 
 def test_scalar_registers_of_large_workgroups():
-    """Large workgroups that share a CU are limited to 80 scalar registers."""
+    """Large workgroups that share a CU are limited to 80 scalar registers;
+    with few groups, or static LDS of more than half a CU, they have it alone."""
+    from dogqc_amd import autotune
+    from dogqc_amd.hipTranslator import staticLdsBytes
+    comp = autotune.translateVariant("tpch2", 1024, 1)
+    alone = [staticLdsBytes(p) > 80 << 10 for p in comp.program.pipes]
+    assert any(alone) and not all(alone)
+    for p, one in zip(comp.program.pipes, alone):
+        assert ("amdgpu_num_sgpr(80))) %s(" % p.name in comp.source) == (not one and p.bs >= 512 and not p.fewGroups)
     few, many, small = planlib.translate("tpch1").source, planlib.translate("tpch18").source, planlib.translate("c1").source
     assert "__launch_bounds__(1024) krnl_lineitem1(" in few
     assert "__launch_bounds__(1024) __attribute__((amdgpu_num_sgpr(80))) krnl_lineitem1(" in many
