@@ -859,7 +859,7 @@ def pipelineLaunch(prog, pipe, phase=None, rowsExpr=None, perCu=8):
         U = 1 if pipe.drains and phase == 1 else pipe.frontU
         lines.append("const unsigned g = gridFor(t->grid[%d] > 0 ? t->grid[%d] : %d, %s, %d, %s, %d, %d);"
                      % (pipe.pipeId, pipe.pipeId, pipe.defaultGrid, rows, pipe.bs, per, U, spread))
-    if pipe.fewGroups:
+    if pipe.fewGroups and not pipe.defaultGrid:
         # rows enough for a workgroup to be worth its flush, every group of
         # its table: 8 per slot (a 246 k-row, 175-group group-by
         # 41 us at 240 workgroups, 25 us at 61)

@@ -231,6 +231,19 @@ def test_join_build_grid(n):
     check("c1", workloadAcc("c1", {"dim": n, "fact": 1 << 16}, seed=n % 97), label="dim=%d" % n)
 
 
+def test_a_programs_default_grid_is_taken(monkeypatch):
+    """KernelCall.defaultGridSize holds for every pipeline that the tuning
+    gives no grid, also those whose grid follows from groups or queues."""
+    from dogqc_amd.kernel import KernelCall
+    for plan in ("c0", "c1_refill", "c2_pushdown", "tpch1"):
+        monkeypatch.setattr(KernelCall, "defaultGridSize", 0)
+        chosen = planlib.translate(plan).source
+        monkeypatch.setattr(KernelCall, "defaultGridSize", 7)
+        asked = planlib.translate(plan).source
+        assert "] <= 0) g = " in chosen and "] <= 0) g = " not in asked, plan
+        assert "] : 7, " in asked and "] : 0, " not in asked
+
+
 def test_scalar_registers_of_large_workgroups():
     """Large workgroups that share a CU are limited to 80 scalar registers;
     with few groups, or static LDS of more than half a CU, they have it alone."""
