@@ -336,8 +336,6 @@ class Pipeline(object):
             else:
                 k.emit("%s %s%s;" % (ct, name, "" if init is None else " = " + init))
         k.extend(self.prologue)
-        # lane refills drain their buffers in one more trip, after the last rows
-        end = "" if self.refillPoints else " base < nrows"
         if U == 1:
             first, step = "(int64_t)blockIdx.x * %d" % B, "(int64_t)gridDim.x * %d" % B
         else:

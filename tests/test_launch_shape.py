@@ -1,6 +1,10 @@
 """Row-to-thread mapping of pipelines with several rows per thread: a table of
 at least one full trip of the grid is walked in tiles, a smaller one in steps
 of the whole grid, and both have to reach every row exactly once."""
+import ctypes
+import re
+import subprocess
+
 import numpy as np
 import pytest
 
@@ -13,36 +17,61 @@ from tests.test_gpu_parity import check, workloadAcc
 GRID = 3
 
 
-def walk(n, grid, B, U):
-    """Rows in the order the generated loop assigns them (Pipeline.render)."""
-    tiled = n >= grid * B * U
-    step, trip = (B if tiled else grid * B), grid * B * U
-    out = []
-    for wg in range(grid):
-        base = wg * (B * U if tiled else B)
-        while base < n:
-            for u in range(U):
-                rows = base + u * step + np.arange(B)
-                out.append(rows[rows < n])
-            base += trip
-    return np.concatenate(out) if out else np.zeros(0, int)
+@pytest.fixture(scope="module")
+def walk(tmp_path_factory):
+    """Rows in the order that the loop of a generated kernel assigns them: its
+    own statements (Pipeline.render), compiled for the host."""
+    built = {}
+
+    def rows(U, n, grid):
+        if U not in built:
+            with planlib.knobs(rowsPerThread=U):
+                comp = planlib.translate("c1", rowsPerThread=U)
+            pipe = comp.program.pipes[0]
+            assert pipe.frontU == U
+            body = comp.source[comp.source.index(" %s(const" % pipe.name):]
+            own = [ln.strip() for ln in body[:body.index("active[u] = more")].splitlines()]
+            head = [ln for ln in own if ln.startswith(("const bool tiled", "const int64_t step"))]
+            loop = [ln for ln in own if ln.startswith("for (int64_t base")]
+            row = [ln for ln in own if ln.startswith("%s[u] = base" % pipe.tid)]
+            assert loop and len(loop) == len(row) == 1
+            d = tmp_path_factory.mktemp("walk")
+            (d / "w.cpp").write_text("""#include <cstdint>
+struct dim { uint32_t x; };
+extern "C" long walk(int64_t nrows, uint32_t grid, int64_t* out) {
+    long n = 0;
+    const dim gridDim{grid};
+    dim blockIdx{0}, threadIdx{0};
+    for (; blockIdx.x < grid; ++blockIdx.x)
+        for (threadIdx.x = 0; threadIdx.x < %du; ++threadIdx.x) {
+            %s
+            %s
+                for (int u = 0; u < %d; ++u) {
+                    int64_t %s[%d];
+                    %s
+                    if (%s[u] < nrows) out[n++] = %s[u];
+                }
+            }
+        }
+    return n;
+}
+""" % (pipe.bs, "\n".join(head), loop[0], U, pipe.tid, U, row[0], pipe.tid, pipe.tid))
+            subprocess.run(["g++", "-O1", "-shared", "-fPIC", str(d / "w.cpp"), "-o", str(d / "w.so")], check=True)
+            built[U] = (ctypes.CDLL(str(d / "w.so")), pipe.bs)
+        lib, _ = built[U]
+        out = np.zeros(2 * n + 1, dtype=np.int64)
+        count = lib.walk(ctypes.c_int64(n), ctypes.c_uint32(grid), out.ctypes.data_as(ctypes.c_void_p))
+        return out[:count], built[U][1]
+    return rows
 
 
 @pytest.mark.parametrize("U", [1, 2, 4])
-def test_every_row_once(U):
-    B = 8
+def test_every_row_once(U, walk):
+    B = walk(U, 1, 1)[1]
     for grid in (1, 3, 4):
         full = grid * B * U
         for n in {0, 1, B - 1, B, B + 1, full - 1, full, full + 1, 2 * full - 1, 2 * full, 2 * full + B + 1}:
-            assert np.array_equal(np.sort(walk(n, grid, B, U)), np.arange(n)), (U, grid, n)
-
-
-def test_rendered_mapping():
-    """The generated kernels carry the mapping that `walk` states."""
-    src = planlib.translate("c0").source
-    assert "const bool tiled = nrows >= (int64_t)gridDim.x * 1024;" in src
-    assert "const int64_t step = tiled ? (int64_t)256 : (int64_t)gridDim.x * 256, trip = (int64_t)gridDim.x * 1024;" in src
-    assert "base = (int64_t)blockIdx.x * (tiled ? 1024 : 256); base < nrows; base += trip" in src
+            assert np.array_equal(np.sort(walk(U, n, grid)[0]), np.arange(n)), (U, grid, n)
 
 
 # one full trip of 3 workgroups x 256 threads x 4 rows is 3072 rows
@@ -119,9 +148,6 @@ def test_default_filter_is_held_in_lds(tmp_path):
     """A filter of a size the plan was translated with goes to LDS like one
     the tuning asks for; the size chosen from the key count does not.  (The
     generated host code's own statements, compiled for the host.)"""
-    import re
-    import subprocess
-
     def words(default, request):
         alg, p, cfg, opts = planlib.build("c3_refill", planlib.emptyAccessor("c3_refill"))
         plan = alg.resolveAlgebraPlan(p, cfg)
@@ -220,8 +246,9 @@ def test_join_builds_take_a_row_per_thread():
     """A pipeline that ends in inserts into a join table is launched on four
     times the workgroups of the others."""
     src = planlib.translate("c1").source
-    host = [ln for ln in src.splitlines() if "gridFor(t->grid[" in ln]
-    assert host[0].split("gridFor")[1].endswith(", 256, 32, 4, 32);") and not any("32, 4, 32" in ln for ln in host[1:])
+    calls = re.findall(r"gridFor\(t->grid[^;]*?,\s*(\d+),\s*(\d+),\s*(\d+),\s*(\d+)\);", src)
+    (_, build, _, spread), others = [int(x) for x in calls[0]], [[int(x) for x in c] for c in calls[1:]]
+    assert others and spread == build and all(build == 4 * perCu for _, perCu, _, _ in others)
 
 
 # the build's grid ends at 256 CUs x 32 workgroups x 256 rows
