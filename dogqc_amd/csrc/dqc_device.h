@@ -1204,8 +1204,10 @@ __device__ inline uint64_t block_excl_scan(uint64_t v, uint64_t* sh, uint64_t& t
     return r;
 }
 
-// One launch, one read and one write of the directory: 1 M buckets 13 us
-// (three launches and two strided reads took 28 us).  A workgroup takes a tile of SCAN_TILE
+// One launch, one read and one write of the directory, where three launches
+// read it twice in strides: 2^20 buckets 28.6 -> 13.5 us from the step before
+// to the step after (19.4 -> 10.5 in the kernels), 2^21 38.3 -> 20.8 (28.8 ->
+// 17.8).  A workgroup takes a tile of SCAN_TILE
 // buckets from the ticket counter state[0], publishes the tile's total in
 // state[1 + tile] and adds up its predecessors' from there (decoupled
 // look-back: Merrill and Garland, "Single-pass Parallel Prefix Scan with
