@@ -47,3 +47,14 @@ def test_nearest_bucket():
     assert autotune.nearest(recs, 1 << 24) == "c"            # tie 22/26 -> the larger bucket
     assert autotune.nearest(recs, 1 << 29) is None           # 3 buckets from the nearest
     assert autotune.nearest({}, 100) is None
+
+
+def test_tracked_records_were_timed_on_their_plans():
+    """A record lists the times of exactly the launches its plan now has: a
+    record pointed at another plan source without a search does not."""
+    for f in sorted(os.listdir(autotune.CACHE_DIR)):
+        with open(os.path.join(autotune.CACHE_DIR, f)) as fh:
+            rec = json.load(fh)
+        comp = autotune.translateVariant(rec["plan"], rec["block"], rec["rows_per_thread"])
+        assert autotune.planKey(comp.source) == rec["plan_source"], f
+        assert set(rec["kernels_ms"]) - {"_total"} == {s["name"] for s in comp.program.steps}, f
