@@ -2207,11 +2207,12 @@ class AggregationTranslator(UnaryTranslator):
 
         Flushing every group with a claim and an atomic per accumulator took
         277 us for 1.5 M groups of 6 M rows and 94 us for 106 k groups of
-        3.2 M rows; the image takes 68 and 64 us (with 1024 threads a
+        3.2 M rows; the image takes 71 and 64 us (with 1024 threads a
         workgroup; with 256, too few wavefronts for the records' latency, 135
-        and 116).  At 8 k groups of 246 k rows, 70 us unpartitioned, 25 us
-        partitioned; 16 k of 1.1 M, 172 and 58.  Fewer than one partition per
-        CU leaves CUs idle (64 partitions: 25 us in the second launch alone).
+        and 116).  Both launches against the unpartitioned update: 2049 groups
+        of 70 k rows 40 -> 16 us, 2500 of 246 k 69 -> 20, 8 k of 246 k 63 ->
+        22, 16 k of 1.1 M 116 -> 38.  Fewer than one partition per CU leaves
+        CUs idle (64 partitions: 25 us in the second launch alone).
 
         With no partitions (tuning part_agg, or a small or unknown group
         count) PHASE 0 is the plain exact-tag update and PHASE 1 is not
