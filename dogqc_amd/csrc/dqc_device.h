@@ -342,12 +342,15 @@ DQC_DEVICE_INLINE T packed_payload(uint64_t slot) {
 // empty slot before it: with an empty slot in the window and no hit, it is
 // absent.  A slot word's tag is its low half where words are packed slots.
 //
-// VALU instructions bound the probes of streamed rows: c3's sales kernel spent
-// 493 a wavefront and trip (60 M rows, 462 M in all, 1155 us), most of them in
-// 64-bit slot bookkeeping per window slot, in mix64 and in a walk of one slot
-// and memory round trip at a time for the lanes (1 in 8 at a load of one half)
-// whose window does not decide.  With hash32, this window test and a walk by
-// windows it takes 762 us, TPC-H Q3's two probing kernels 125 -> 85 us.
+// VALU instructions bound the probes of streamed rows where every row probes:
+// c3's sales kernel spent 493 a wavefront and trip (60 M rows, 462 M in all,
+// two thirds of the SIMDs' cycles in 1155 us), most of them in 64-bit slot
+// bookkeeping per window slot, in mix64 and in a walk of one slot and memory
+// round trip at a time for the lanes (1 in 8 at a load of one half) whose
+// window does not decide.  With hash32, this window test and a walk by windows
+// it took 762 us, TPC-H Q3's two probing kernels 125 -> 85 us.  (Tuned and
+// behind a filter and a lane refill the kernel now issues 47 M, one sixth of
+// the cycles, and waits for memory.)
 template <typename Slot, typename Tag>
 DQC_DEVICE_INLINE uint32_t window_find(const probe_win<Slot>& w, Tag tag, bool& empty) {
     uint32_t k = PROBE_WINDOW;
@@ -1082,7 +1085,8 @@ DQC_DEVICE_INLINE bool bytes_equal(const char* a, const char* b, uint32_t n) {
 // `head` holds lit's first H = min(L, 8) bytes, lit[k] in bits 8k and up.
 //
 // The string's aligned words are loaded eight at a time (independent loads,
-// one round trip for 56 start positions).  VALU instructions bound the search,
+// one round trip for 56 start positions).  VALU instructions bound the search
+// (64 to 70 % of the SIMDs' cycles still issue one),
 // so four positions share each: dword j shifted by k bytes holds byte k after
 // them (v_alignbyte), and a zero byte in the OR of its differences to lit[k]
 // is a match of all H bytes.  About 12 instructions per 4 positions for a
