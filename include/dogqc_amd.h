@@ -90,8 +90,8 @@ typedef struct dqc_plan_tuning {
                                                 into dqc_plan_status.ht_fill after the plan */
     int32_t part_agg;                        /* partitioned group-by (plans translated with it): 0 = when
                                                 the group count (ht_capacity / 2, else the plan's numgroups)
-                                                exceeds 2048 and the input 65536 rows, -1 = never,
-                                                n > 0 = n partitions */
+                                                exceeds 2048 and 65536 rows or more are estimated
+                                                to reach it, -1 = never, n > 0 = n partitions */
     int32_t join_filter;                     /* filter of the build keys of selective unique joins: n > 0 =
                                                 n KB (in LDS when it fits), 0 = the size the plan was
                                                 translated with, else 16 bits per key in device memory for
